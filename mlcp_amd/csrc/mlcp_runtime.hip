@@ -15,6 +15,7 @@
 //   download block.
 // Everything runs on one non-default stream of default priority.
 #include "mlcp_kernels.hip"
+#include "mlcp_gs.hip"
 #include "mlcp_mlp.hip"
 #include <hip/hip_ext.h>
 #include <dlfcn.h>
@@ -25,6 +26,8 @@
 #include <cstdlib>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -122,8 +125,9 @@ static int nx_of(int nmax) {
   return need <= 8 ? 8 : need <= 12 ? 12 : need <= 16 ? 16 : need <= 24 ? 24 : 32;
 }
 
-// LDS per workgroup of the device (static plus dynamic).
+// LDS per workgroup of the device (static plus dynamic), and its CUs.
 static size_t g_lds_dev = 64 * 1024;
+static int g_cus = 1;
 
 static int setup_kernels() {
   static bool done = false;
@@ -131,6 +135,8 @@ static int setup_kernels() {
   int dev = 0, v = 0;
   HCHK(hipGetDevice(&dev));
   HCHK(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock,
+                             dev));
+  HCHK(hipDeviceGetAttribute(&g_cus, hipDeviceAttributeMultiprocessorCount,
                              dev));
 #define NX_KERNELS(kern)                                                    \
   (const void*)kern<8>, (const void*)kern<12>, (const void*)kern<16>,       \
@@ -144,6 +150,8 @@ static int setup_kernels() {
                       NX_KERNELS(k_gs_terms),
                       NX_KERNELS2(k_gs_reduce, 1), NX_KERNELS2(k_gs_reduce, 2),
                       NX_KERNELS2(k_gs_reduce, 3), NX_KERNELS2(k_gs_reduce, 4),
+                      NX_KERNELS2(k_gs_state, 1), NX_KERNELS2(k_gs_state, 2),
+                      NX_KERNELS2(k_gs_state, 3), NX_KERNELS2(k_gs_state, 4),
                       NX_KERNELS2(k_op_solve, 1),  NX_KERNELS2(k_op_solve, 2),
                       NX_KERNELS2(k_op_solve, 3),  NX_KERNELS2(k_op_solve, 4),
                       (const void*)k_lc_solve<1>,  (const void*)k_lc_solve<2>,
@@ -222,6 +230,16 @@ struct mlcp_session {
   // Gram-Schmidt
   DBuf<double> gsX, gsXS, gsG, gsPart, gsBbs, gsPc, gsBjk, gsGjf;
   DBuf<int> gsCnt;
+  // one launch per state (k_gs_state): parts, solution and stop words, the
+  // product caches, first step number and the flag of a wait that ran out
+  DBuf<u64> gsP, gsLX, gsCtrl;
+  DBuf<double> gsT, gsS;
+  DBuf<unsigned> gsEp;
+  DBuf<int> gsAb;
+  int gs_nS = -1, gs_SL = 0;   // its slice workgroups (0: not used, -1: not yet set)
+  bool gs_steps = false;    // kernel-per-step form for this call
+  bool gs_timeout = false;  // a wait of the last call ran out
+  std::shared_ptr<struct GsEvent> gs_ev;
   // form of the cycle (mlcp_hip_session_set_form): bit 1 = ALS phases to a
   // residual tolerance instead of the fixed sweep counts
   int form = 0;
@@ -546,13 +564,56 @@ static int build_had_jobs(mlcp_session* s) {
   return 0;
 }
 
+// Shape and buffers of the one-launch-per-state Gram-Schmidt (k_gs_state): a
+// slice workgroup for every column of the largest mode, for every two columns
+// from 65 on (a quarter of the CUs at most), a term workgroup on a CU of its
+// own for every previous state.  Devices that
+// cannot hold both at once (a partition with fewer CUs) keep the
+// kernel-per-step form, and so does a session of one drop-in call: that call
+// returns the block itself, and the factors of a block amplify rounding (a
+// last-bit change before the eigenproblem moves them by 1e-10, for some blocks
+// of three modes by 3e-9), so its results stay the bits they have been.
+static size_t gs_slw(int RTM) { return (size_t)RTM * (RTM >= 3 ? 4 : 2) * 256; }
+
+static int gs_alloc(mlcp_session* s) {
+  const int B = s->nbloc, D = s->ndof;
+  if (s->gs_nS >= 0) return 0;
+  s->gs_nS = 0;
+  if (B < 2 || s->oneshot) return 0;
+  const int nS0 = std::min(s->nmax, g_cus / 4);
+  if (nS0 < 1) return 0;
+  const int SL = (s->nmax + nS0 - 1) / nS0, nS = (s->nmax + SL - 1) / SL;
+  if (SL > GS_SLMAX || g_cus - nS < 32) return 0;
+  const int RTM = (s->Rmax + 15) / 16;
+  const size_t slw = gs_slw(RTM);
+  const size_t step = 2 * (size_t)s->nmax * s->Rmax;
+  if (s->gsP.need((size_t)(B - 1) * (step + 2)) || s->gsLX.need(2 * step) ||
+      s->gsCtrl.need(2) || s->gsT.need((size_t)(B - 1) * D * slw) ||
+      s->gsS.need((size_t)nS * D * slw) || s->gsEp.need(1) ||
+      s->gsAb.need(1))
+    return -1;
+  // step numbers start at 1, so cleared words belong to no step
+  hipLaunchKernelGGL(k_fill, dim3(256), dim3(256), 0, s->st,
+                     (double*)s->gsP.p, (long)((B - 1) * (step + 2)), 0.0);
+  hipLaunchKernelGGL(k_fill, dim3(64), dim3(256), 0, s->st,
+                     (double*)s->gsLX.p, (long)(2 * step), 0.0);
+  hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, s->st,
+                     (double*)s->gsCtrl.p, 2L, 0.0);
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s->st,
+                     (int*)s->gsEp.p, 1L, 1);
+  HCHK(hipGetLastError());
+  s->gs_nS = nS;
+  s->gs_SL = SL;
+  return 0;
+}
+
 static int session_alloc(mlcp_session* s) {
   int D = s->ndof, B = s->nbloc;
   hipStream_t st = s->st;
   int rstr = s->Rmax * s->Rmax;
   int ystr = s->nmax * s->Rmax;
-  // pool: three regions of Ntot columns
-  int cap = 3 * s->Ntot;
+  // pool: four regions of Ntot columns
+  int cap = 4 * s->Ntot;
   if (s->fac.need((size_t)cap * s->nD) || s->coef.need(cap) ||
       s->err.need(1))
     return -1;
@@ -609,15 +670,10 @@ static int session_alloc(mlcp_session* s) {
   s->had_split = 4;
   s->gs_xst = gs_stride();
   if (build_had_jobs(s)) return -1;
-  // Gram-Schmidt
-  int pstr = s->Rmax * s->nmax;
-  if (s->gsX.need((size_t)B * D * rstr) || s->gsXS.need((size_t)B * D * rstr) ||
-      s->gsG.need((size_t)D * rstr) ||
-      s->gsPart.need((size_t)(B + 1) * pstr) || s->gsBbs.need(rstr) ||
-      s->gsPc.need((size_t)(B + 1) * GS_PCS) || s->gsBjk.need(pstr) ||
-      s->gsGjf.need(GJF_SIZE) || s->gsCnt.need(1) || s->gsDone.need(B) ||
-      s->opDone.need(B) || s->lcDone.need(B) || s->opPrev.need(B) ||
-      s->lcPrev.need(B))
+  // state of the tolerance form (the Gram-Schmidt buffers: gs_alloc,
+  // gs_steps_alloc)
+  if (s->gsDone.need(B) || s->opDone.need(B) || s->lcDone.need(B) ||
+      s->opPrev.need(B) || s->lcPrev.need(B))
     return -1;
   // GEP
   std::vector<PairJob> pj;
@@ -724,6 +780,10 @@ static int check_err(mlcp_session* s, const char* phase) {
   HCHK(hipMemcpyAsync(&e, s->err.p, sizeof(int), hipMemcpyDeviceToHost,
                       s->st));
   HCHK(hipStreamSynchronize(s->st));
+  if (e & 16) {   // run again in the kernel-per-step form (gs_retry)
+    s->gs_timeout = true;
+    return fail(std::string(phase) + ": a Gram-Schmidt hand-over ran out");
+  }
   if (e) {
     std::string m = std::string(phase) + ": ";
     if (e & 1) m += "NaN or zero norm on update; ";
@@ -785,7 +845,7 @@ static int check_err(mlcp_session* s, const char* phase) {
 enum {
   KID_OP_HADAMARD = 1, KID_OP_SOLVE, KID_OP_REFRESH, KID_GS_TERMS,
   KID_GS_REDUCE, KID_LC_RHS, KID_LC_SOLVE, KID_LC_REFRESH, KID_PAIR_INNER,
-  KID_GEP
+  KID_GEP, KID_GS_STATE
 };
 
 // Start/stop events of the next launch of kernel kid while it is probed
@@ -951,57 +1011,185 @@ static GsArgs gs_args(mlcp_session* s, int iv) {
   return g;
 }
 
-static int launch_ortho(mlcp_session* s, int nals);
-
 // Graph replay is the default; MLCP_HIP_GRAPH=0 launches kernel by kernel.
 static bool use_graphs() {
   const char* e = getenv("MLCP_HIP_GRAPH");
   return !(e && e[0] == '0');
 }
 
-static int phase_ortho(mlcp_session* s, int nals) {
-  if (nals < 1) return 0;
-  bool probing = s->probe_kid == KID_GS_TERMS || s->probe_kid == KID_GS_REDUCE;
-  if (!use_graphs() || probing || s->oneshot || s->capturing)
-    return launch_ortho(s, nals);
-  if (!s->gs_exec || s->gs_nals != nals) {
-    if (s->gs_exec) {
-      HCHK(hipGraphExecDestroy(s->gs_exec));
-      s->gs_exec = nullptr;
-    }
-    hipGraph_t g = nullptr;
-    HCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-    int rc = launch_ortho(s, nals);
-    hipError_t e = hipStreamEndCapture(s->st, &g);
-    if (rc) return -1;
-    if (e != hipSuccess)
-      return fail(std::string("gram-schmidt capture: ") + hipGetErrorString(e));
-    e = hipGraphInstantiate(&s->gs_exec, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    if (e != hipSuccess)
-      return fail(std::string("gram-schmidt instantiate: ") +
-                  hipGetErrorString(e));
-    s->gs_nals = nals;
+// Polls a wait of k_gs_state makes before it gives up (each takes at least
+// half a microsecond); MLCP_HIP_GS_SPIN sets it, 0 selects the
+// kernel-per-step form.
+static int gs_spin() {
+  const char* e = getenv("MLCP_HIP_GS_SPIN");
+  return e ? std::max(0, atoi(e)) : 1 << 20;
+}
+
+static bool gs_one_launch(mlcp_session* s) {
+  const bool probing =
+      s->probe_kid == KID_GS_TERMS || s->probe_kid == KID_GS_REDUCE;
+  return s->gs_nS > 0 && !s->gs_steps && !probing && gs_spin() > 0;
+}
+
+// The workgroups of k_gs_state wait for each other, so all of a grid has to
+// be resident: one grid fits by its size, two might not.  Sessions of one
+// process therefore take turns on a device: each phase waits, on the GPU, for
+// the event the last one recorded.  (Another process's grid can still be in
+// the way; the waits are bounded, and the call is then run again in the
+// kernel-per-step form.)
+struct GsEvent {
+  hipEvent_t e = nullptr;
+  ~GsEvent() {
+    if (e) (void)hipEventDestroy(e);
   }
-  HCHK(hipGraphLaunch(s->gs_exec, s->st));
+};
+
+struct GsTurn {
+  static constexpr int MAXDEV = 64;
+  static std::mutex& mu() {
+    static std::mutex* m = new std::mutex;   // never destroyed: used at exit
+    return *m;
+  }
+  static std::shared_ptr<GsEvent>* last() {
+    static auto* l = new std::shared_ptr<GsEvent>[MAXDEV];
+    return l;
+  }
+  std::unique_lock<std::mutex> lock{mu()};
+  int dev = 0;
+  int begin(mlcp_session* s) {
+    HCHK(hipGetDevice(&dev));
+    if (dev < 0 || dev >= MAXDEV) return fail("device index out of range");
+    if (!s->gs_ev) {
+      s->gs_ev = std::make_shared<GsEvent>();
+      HCHK(hipEventCreateWithFlags(&s->gs_ev->e, hipEventDisableTiming));
+    }
+    std::shared_ptr<GsEvent>& l = last()[dev];
+    if (l && l != s->gs_ev) HCHK(hipStreamWaitEvent(s->st, l->e, 0));
+    return 0;
+  }
+  int end(mlcp_session* s) {
+    HCHK(hipEventRecord(s->gs_ev->e, s->st));
+    last()[dev] = s->gs_ev;
+    return 0;
+  }
+};
+
+#define GS_STATE_LAUNCH(RTM)                                                \
+  do {                                                                      \
+    switch (nx) {                                                           \
+      case 8: GS_STATE_NX(8, RTM); break;                                   \
+      case 12: GS_STATE_NX(12, RTM); break;                                 \
+      case 16: GS_STATE_NX(16, RTM); break;                                 \
+      case 24: GS_STATE_NX(24, RTM); break;                                 \
+      default: GS_STATE_NX(32, RTM);                                        \
+    }                                                                       \
+  } while (0)
+#define GS_STATE_NX(nx_, RTM)                                               \
+  PLAUNCH(KID_GS_STATE, (k_gs_state<nx_, RTM>), grid, dim3(GS_NT), lds, g)
+
+// Dynamic LDS of k_gs_state (the layout at its top).
+static size_t gs_state_lds(int nx, int RTM, int D) {
+  const size_t rp = 16 * RTM, xst = 4 * nx + 2;
+  const size_t bst = (RTM & 1) ? rp : rp + 16;
+  return (std::max(rp * xst, (rp + 1) * (rp + 18)) + rp * std::max(bst, rp + 1) +
+          2 * GS_NT + (size_t)(D + 1) * 64 * GS_SLMAX) * sizeof(double);
+}
+
+static int gs_steps_alloc(mlcp_session* s);
+static int launch_ortho_steps(mlcp_session* s, int nals, int iv0);
+
+static int launch_ortho_states(mlcp_session* s, int nals) {
+  const int D = s->ndof, B = s->nbloc, nx = nx_of(s->nmax);
+  const int RTM = (s->Rmax + 15) / 16, nst = nals * D;
+  const size_t lds = gs_state_lds(nx, RTM, D);
+  const unsigned per = (unsigned)nst + 2;
+  const int spin = gs_spin();
+  hipLaunchKernelGGL(k_gs_begin, dim3(1), dim3(256), 0, s->st, s->gsEp.p,
+                     per * (unsigned)B, s->gsAb.p, s->gsDone.p, B);
+  hipLaunchKernelGGL(k_normcoef, dim3(1), dim3(MLCP_NT), 0, s->st, s->pool,
+                     s->roff[0], s->ranks[0]);
+  hipLaunchKernelGGL(k_penalty, dim3((B + 63) / 64), dim3(64), 0, s->st,
+                     s->pool, s->d_colQ.p, s->d_R.p, 1.e-10, s->d_pen.p, B);
+  GsRun g;
+  g.p = s->pool;
+  g.nals = nals;
+  g.col = s->d_colQ.p;
+  g.Rl = s->d_R.p;
+  g.nS = s->gs_nS;
+  g.SL = s->gs_SL;
+  g.P = s->gsP.p;
+  g.X = s->gsLX.p;
+  g.xstr = 2 * (long)s->nmax * s->Rmax;
+  g.pstr = g.xstr + 2;
+  g.ctrl = s->gsCtrl.p;
+  g.tsl = s->gsT.p;
+  g.ssl = s->gsS.p;
+  g.slw = (long)gs_slw(RTM);
+  g.ebase = s->gsEp.p;
+  g.ab = s->gsAb.p;
+  g.spin = spin;
+  g.err = s->err.p;
+  g.done = (s->form & FORM_TOL) ? s->gsDone.p : nullptr;
+  g.tol2 = s->gs_tol * s->gs_tol;
+  // the states that have a CU for every previous one; the kernel-per-step
+  // form takes the others
+  const int last = std::min(B, g_cus - g.nS + 1);
+  for (int iv = 1; iv < last; iv++) {
+    g.iv = iv;
+    g.R = s->ranks[iv];
+    g.cF = s->roff[iv];
+    g.pen = s->d_pen.p + iv;
+    // numbers ebase - per B + per iv + 1 ..: past the last phase's, which
+    // ended below ebase
+    g.eoff = per * (unsigned)iv - per * (unsigned)B;
+    const dim3 grid(g.nS + iv);
+    if (RTM == 1) GS_STATE_LAUNCH(1);
+    else if (RTM == 2) GS_STATE_LAUNCH(2);
+    else if (RTM == 3) GS_STATE_LAUNCH(3);
+    else GS_STATE_LAUNCH(4);
+  }
+  if (last < B && (gs_steps_alloc(s) || launch_ortho_steps(s, nals, last)))
+    return -1;
+  hipLaunchKernelGGL(k_gs_end, dim3(1), dim3(64), 0, s->st,
+                     (const int*)s->gsAb.p, s->err.p);
+  HCHK(hipGetLastError());
   return 0;
 }
 
-static int launch_ortho(mlcp_session* s, int nals) {
+// The kernel-per-step form: two launches per step.  It runs where the device
+// cannot hold the one-launch form's workgroups, where its kernels are probed,
+// and again for a call in which a hand-over of that form ran out.
+static int gs_steps_alloc(mlcp_session* s) {
+  const int D = s->ndof, B = s->nbloc;
+  const int rstr = s->Rmax * s->Rmax, pstr = s->Rmax * s->nmax;
+  if (s->gsX.need((size_t)B * D * rstr) || s->gsXS.need((size_t)B * D * rstr) ||
+      s->gsG.need((size_t)D * rstr) ||
+      s->gsPart.need((size_t)(B + 1) * pstr) || s->gsBbs.need(rstr) ||
+      s->gsPc.need((size_t)(B + 1) * GS_PCS) || s->gsBjk.need(pstr) ||
+      s->gsGjf.need(GJF_SIZE) || s->gsCnt.need(1))
+    return -1;
+  return 0;
+}
+
+// States iv0.. of the block (iv0 > 0: the rest of a phase begun in the
+// one-launch form).
+static int launch_ortho_steps(mlcp_session* s, int nals, int iv0) {
   int D = s->ndof;
   // the done-counter of k_gs_reduce starts every phase at zero (a fill
   // kernel, so the phase can be captured)
   hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s->st, s->gsCnt.p, 1L, 0);
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, s->st, s->gsDone.p,
-                     (long)s->nbloc, 0);
-  hipLaunchKernelGGL(k_normcoef, dim3(1), dim3(MLCP_NT), 0, s->st, s->pool,
-                     s->roff[0], s->ranks[0]);
-  hipLaunchKernelGGL(k_penalty, dim3((s->nbloc + 63) / 64), dim3(64), 0,
-                     s->st, s->pool, s->d_colQ.p, s->d_R.p, 1.e-10,
-                     s->d_pen.p, s->nbloc);
+  if (iv0 == 0) {
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, s->st, s->gsDone.p,
+                       (long)s->nbloc, 0);
+    hipLaunchKernelGGL(k_normcoef, dim3(1), dim3(MLCP_NT), 0, s->st, s->pool,
+                       s->roff[0], s->ranks[0]);
+    hipLaunchKernelGGL(k_penalty, dim3((s->nbloc + 63) / 64), dim3(64), 0,
+                       s->st, s->pool, s->d_colQ.p, s->d_R.p, 1.e-10,
+                       s->d_pen.p, s->nbloc);
+  }
   // k_gs_terms: four waves' partial P tiles, 4 * (NX / 4) * 256 doubles
   const size_t lds_t = (size_t)256 * nx_of(s->nmax) * sizeof(double);
-  for (int iv = 1; iv < s->nbloc; iv++) {
+  for (int iv = std::max(1, iv0); iv < s->nbloc; iv++) {
     GsArgs g = gs_args(s, iv);
     int kprev = -1;
     int nch = (s->ranks[iv] + GS_ICH - 1) / GS_ICH;
@@ -1028,6 +1216,40 @@ static int launch_ortho(mlcp_session* s, int nals) {
       }
   }
   HCHK(hipGetLastError());
+  return 0;
+}
+
+static int phase_ortho(mlcp_session* s, int nals) {
+  if (nals < 1) return 0;
+  if (gs_one_launch(s)) {
+    if (s->capturing) return launch_ortho_states(s, nals);
+    GsTurn turn;
+    return turn.begin(s) || launch_ortho_states(s, nals) || turn.end(s) ? -1 : 0;
+  }
+  if (gs_steps_alloc(s)) return -1;   // before a capture begins
+  bool probing = s->probe_kid == KID_GS_TERMS || s->probe_kid == KID_GS_REDUCE;
+  if (!use_graphs() || probing || s->oneshot || s->capturing || s->gs_steps)
+    return launch_ortho_steps(s, nals, 0);
+  if (!s->gs_exec || s->gs_nals != nals) {
+    if (s->gs_exec) {
+      HCHK(hipGraphExecDestroy(s->gs_exec));
+      s->gs_exec = nullptr;
+    }
+    hipGraph_t g = nullptr;
+    HCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
+    int rc = launch_ortho_steps(s, nals, 0);
+    hipError_t e = hipStreamEndCapture(s->st, &g);
+    if (rc) return -1;
+    if (e != hipSuccess)
+      return fail(std::string("gram-schmidt capture: ") + hipGetErrorString(e));
+    e = hipGraphInstantiate(&s->gs_exec, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (e != hipSuccess)
+      return fail(std::string("gram-schmidt instantiate: ") +
+                  hipGetErrorString(e));
+    s->gs_nals = nals;
+  }
+  HCHK(hipGraphLaunch(s->gs_exec, s->st));
   return 0;
 }
 
@@ -1188,8 +1410,31 @@ static int phase_update(mlcp_session* s, const double* Ud, int nals) {
   return lc_als(s, a, nals, true);
 }
 
-static int run_cycle(mlcp_session* s, double* eigv, int npow, int nals,
-                     int update, int ishift, double eshift) {
+// Runs a call f that holds a Gram-Schmidt phase; if a hand-over of the
+// one-launch form ran out (the device is shared with a process that keeps
+// some of its workgroups out), the block is put back and the call runs again
+// in the kernel-per-step form.
+template <class F>
+static int gs_retry(mlcp_session* s, F f) {
+  if (gs_alloc(s)) return -1;
+  if (!gs_one_launch(s)) return f();
+  const int N = s->Ntot;
+  hipLaunchKernelGGL(k_copy_cols, dim3(256), dim3(256), 0, s->st, s->pool, 0,
+                     3 * N, N);
+  s->gs_timeout = false;
+  int rc = f();
+  if (!rc || !s->gs_timeout) return rc;
+  g_err.clear();
+  hipLaunchKernelGGL(k_copy_cols, dim3(256), dim3(256), 0, s->st, s->pool,
+                     3 * N, 0, N);
+  s->gs_steps = true;
+  rc = f();
+  s->gs_steps = false;
+  return rc;
+}
+
+static int run_cycle_once(mlcp_session* s, double* eigv, int npow, int nals,
+                          int update, int ishift, double eshift) {
   hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s->st, s->err.p, 1L, 0);
   HCHK(hipEventRecord(s->ev[0], s->st));
   if (phase_power(s, npow, ishift, eshift)) return -1;
@@ -1217,6 +1462,12 @@ static int run_cycle(mlcp_session* s, double* eigv, int npow, int nals,
   return 0;
 }
 
+static int run_cycle(mlcp_session* s, double* eigv, int npow, int nals,
+                     int update, int ishift, double eshift) {
+  return gs_retry(s, [&] {
+    return run_cycle_once(s, eigv, npow, nals, update, ishift, eshift);
+  });
+}
 
 // --------------------------------------------------------------------------
 // Learned warm start: the MLP of mlcp_mlp.hip, its training and inference.
@@ -1554,10 +1805,9 @@ static int solve_cycle_body(mlcp_session* s, int npow, int nals, double lo,
   return 0;
 }
 
-extern "C" int mlcp_hip_session_solve(mlcp_session* s, double* eigv,
-                                      const double* bounds, int ncycle,
-                                      int npow, int nals, double* hist) {
-  g_err.clear();
+static int session_solve_once(mlcp_session* s, double* eigv,
+                              const double* bounds, int ncycle, int npow,
+                              int nals, double* hist) {
   const int B = s->nbloc;
   if (ncycle < 1 || npow < 1 || nals < 1)
     return fail("solve: ncycle, npow and nals must be positive");
@@ -1578,9 +1828,10 @@ extern "C" int mlcp_hip_session_solve(mlcp_session* s, double* eigv,
   if (solve_cycle_body(s, npow, nals, lo, hi, ncycle)) return -1;
   const bool graph = use_graphs() && s->probe_kid == 0 && ncycle > 1;
   if (graph) {
-    char key[160];
-    snprintf(key, sizeof key, "%d/%d/%.17g/%.17g/%d/%d/%.17g/%.17g", npow,
-             nals, lo, hi, ncycle, s->form, s->gs_tol, s->als_tol);
+    char key[192];
+    snprintf(key, sizeof key, "%d/%d/%.17g/%.17g/%d/%d/%.17g/%.17g/%d", npow,
+             nals, lo, hi, ncycle, s->form, s->gs_tol, s->als_tol,
+             gs_one_launch(s) ? gs_spin() : 0);
     if (!s->cyc_exec || s->cyc_key != key) {
       if (s->cyc_exec) {
         HCHK(hipGraphExecDestroy(s->cyc_exec));
@@ -1604,7 +1855,14 @@ extern "C" int mlcp_hip_session_solve(mlcp_session* s, double* eigv,
         return fail(std::string("cycle instantiate: ") + hipGetErrorString(e));
       s->cyc_key = key;
     }
-    for (int c = 1; c < ncycle; c++) HCHK(hipGraphLaunch(s->cyc_exec, s->st));
+    if (gs_one_launch(s)) {
+      GsTurn turn;
+      if (turn.begin(s)) return -1;
+      for (int c = 1; c < ncycle; c++) HCHK(hipGraphLaunch(s->cyc_exec, s->st));
+      if (turn.end(s)) return -1;
+    } else {
+      for (int c = 1; c < ncycle; c++) HCHK(hipGraphLaunch(s->cyc_exec, s->st));
+    }
   } else {
     for (int c = 1; c < ncycle; c++)
       if (solve_cycle_body(s, npow, nals, lo, hi, ncycle)) return -1;
@@ -1618,6 +1876,15 @@ extern "C" int mlcp_hip_session_solve(mlcp_session* s, double* eigv,
   HCHK(hipStreamSynchronize(s->st));
   if (hist) memcpy(hist, h.data(), sizeof(double) * h.size());
   return 0;
+}
+
+extern "C" int mlcp_hip_session_solve(mlcp_session* s, double* eigv,
+                                      const double* bounds, int ncycle,
+                                      int npow, int nals, double* hist) {
+  g_err.clear();
+  return gs_retry(s, [&] {
+    return session_solve_once(s, eigv, bounds, ncycle, npow, nals, hist);
+  });
 }
 
 // --------------------------------------------------------------------------
@@ -1977,9 +2244,12 @@ extern "C" int mlcp_hip_session_rayleigh(mlcp_session* s, double* rq) {
 
 extern "C" int mlcp_hip_session_ortho(mlcp_session* s, int nals) {
   g_err.clear();
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s->st, s->err.p, 1L, 0);
-  if (phase_ortho(s, nals)) return -1;
-  return check_err(s, "gram-schmidt");
+  return gs_retry(s, [&] {
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s->st, s->err.p, 1L,
+                       0);
+    if (phase_ortho(s, nals)) return -1;
+    return check_err(s, "gram-schmidt");
+  });
 }
 
 extern "C" int mlcp_hip_session_prodhv(mlcp_session* s, int nals,
@@ -2360,8 +2630,8 @@ extern "C" void intwdevicemem_(const int* rk, const int* ndof,
     nmax = std::max<double>(nmax, nbas[d]);
   }
   const double MB = 1.0 / (1 << 20), N = R * B, r2 = R * R;
-  // pool (3 regions), coefficients, per-state tables, penalties
-  const double pool = 8 * (3 * N * nD + 3 * N) + 4 * (3 * B + N) + 8 * B;
+  // pool (4 regions), coefficients, per-state tables, penalties
+  const double pool = 8 * (4 * N * nD + 4 * N) + 4 * (3 * B + N) + 8 * B;
   // dense operators (n_max^2 bound), term tables and Hadamard records
   const double terms = 8 * O * nmax * nmax + 8 * T + 4 * T * D * 6 +
                        8 * T * 3 + 16 * T * D;
@@ -2369,9 +2639,16 @@ extern "C" void intwdevicemem_(const int* rk, const int* ndof,
   const double opals = 8 * (B * O * r2 + B * D * r2 + B * O * nmax * R +
                             B * O * r2 + B * r2) +
                        8 * (2 * B * (O + D) + B * ((r2 + 63) / 64) * D * 4);
-  // Gram-Schmidt caches (cross Grams and their prefix / suffix products)
-  const double gs = 8 * (2 * B * D * r2 + D * r2 + (B + 1) * R * nmax + r2 +
-                         (B + 1) * GS_PCS + R * nmax + GJF_SIZE) + 4;
+  // Gram-Schmidt: product caches of the previous states and the slices,
+  // parts and solution words (as gs_alloc on a device of 256 CUs)
+  const double t2 = (double)gs_slw((int)std::ceil(R / 16));
+  const double nS = nmax > 64 ? std::ceil(nmax / 2) : nmax;
+  const double gs1 = B < 2 ? 0.0
+      : 8 * ((B - 1 + nS) * D * t2 + (B - 1) * (2 * R * nmax + 2) + 4 * R * nmax + 4);
+  // or the kernel-per-step form's cross Grams, products and partial sums
+  const double gs = std::max(
+      gs1, 8 * (2 * B * D * r2 + D * r2 + (B + 1) * R * nmax + r2 +
+                (B + 1) * GS_PCS + R * nmax + GJF_SIZE) + 4);
   // pair jobs, QHQ and S, U, eigenvalues, eigensolver work
   const double gep = 24.0 * B * (B + 1) + 8 * (2 * B * B + B * B + B +
                                               4 * B * B + 2 * B + 8);
@@ -2382,7 +2659,7 @@ extern "C" void intwdevicemem_(const int* rk, const int* ndof,
             8 * B * std::ceil(N / LC_CHUNK)
       : 0.0;
   printf(" *** MI355X device memory requirements *** \n \n");
-  printf(" Factor pool (3 regions)  : %10.2f MB \n", pool * MB);
+  printf(" Factor pool (4 regions)  : %10.2f MB \n", pool * MB);
   printf(" Term list (dense ops)    : %10.2f MB \n", terms * MB);
   printf(" Operator-ALS caches      : %10.2f MB \n", opals * MB);
   printf(" Gram-Schmidt caches      : %10.2f MB \n", gs * MB);

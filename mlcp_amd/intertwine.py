@@ -192,7 +192,7 @@ class Session:
 
     KERNELS = {"op_hadamard": 1, "op_solve": 2, "op_refresh": 3,
                "gs_terms": 4, "gs_reduce": 5, "lc_rhs": 6, "lc_solve": 7,
-               "lc_refresh": 8, "pair_inner": 9, "gep": 10}
+               "lc_refresh": 8, "pair_inner": 9, "gep": 10, "gs_state": 11}
 
     def probe(self, kernel: str, max_launches: int = 16384):
         kid = self.KERNELS[kernel] if kernel else 0
