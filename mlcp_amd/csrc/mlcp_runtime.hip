@@ -527,6 +527,26 @@ static int had_tile_max(mlcp_session* s) {
   return 0;
 }
 
+// Waves (parts) that share one 64-element group of the Hadamard.  A CU holds
+// sixteen of its waves (by registers), in as many workgroups as their LDS and
+// the number of tiles allow, so the split makes up the sixteen: 200 states of
+// rank 16-64 and 6807 terms fill the LDS with one workgroup, 4 waves take 5.81
+// ms and 16 take 3.03; 120 of rank 32 and 1008 terms fit two, 262 / 195 / 241
+// us for 4 / 8 / 16; 64 of rank 8-48 and 182 terms fit five, 40 / 35 / 48 for
+// 2 / 4 / 8; two states of rank 32 have 32 tiles for 256 CUs, 60 / 43 / 32 for
+// 4 / 8 / 16.  Every part keeps about six records or more (40 states of rank 20
+// and 31 terms: 10.2 us with 4 waves, 11.1 with 8).
+static int had_split_default(mlcp_session* s) {
+  const size_t lds = (size_t)(s->nops + 1 + s->nsubmax) * 64 * sizeof(double);
+  long tiles = 0;
+  for (int R : s->ranks) tiles += (R * R + 63) / 64;
+  const long fit = (long)(lds_limit((const void*)k_op_hadamard) / lds);
+  const long wgs = std::max(1L, std::min(fit, (tiles + g_cus - 1) / g_cus));
+  int P = 1;
+  while (P * wgs < 16 && P < 16 && 12L * P <= s->T) P *= 2;
+  return P;
+}
+
 // Hadamard jobs (state, tile of had_tile elements; a workgroup runs
 // had_tile/64 x had_split waves) and, per mode, the sub-slot ranges of the
 // parts: contiguous sub-slots with about equal record counts.
@@ -661,13 +681,12 @@ static int session_alloc(mlcp_session* s) {
   if (s->jobs_all.put(all, st)) return -1;
   // Hadamard tile: elements per workgroup such that every operator's Gram
   // of the tile (and the entry holding 1) fits in LDS
-  // default: one 64-element group shared by four waves (parts); the
-  // autotuner may choose otherwise
+  // (the autotuner may choose otherwise)
   if (had_tile_max(s) < 64)
     return fail("too many operators (" + std::to_string(s->nops) +
                 ") for the LDS of one workgroup");
   s->had_tile = 64;
-  s->had_split = 4;
+  s->had_split = had_split_default(s);
   s->gs_xst = gs_stride();
   if (build_had_jobs(s)) return -1;
   // state of the tolerance form (the Gram-Schmidt buffers: gs_alloc,
