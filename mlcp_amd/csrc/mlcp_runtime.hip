@@ -1495,9 +1495,11 @@ struct mlcp_mlp {
   MlpDims m;
   hipStream_t st = nullptr;
   DBuf<float> P, G, Mo, Vo;          // parameters, gradients, Adam moments
-  DBuf<float> X0, Z1, Z2, Y, dY, dH2, dH1, dX0;   // batch work (nbmax rows)
+  DBuf<float> X0, Z1, Z2, Y, dY, dH2, dH1, dXe;   // batch work (nbmax rows)
+  DBuf<float> part;                  // gradients by ranges of batch rows
   DBuf<double> sse;
   int nbmax = 0;
+  int cus = 1;                       // CUs of the device
   int step = 0;                      // Adam steps taken
   // training set (device) and warm-start inputs
   DBuf<float> tX, tT, wX, wY;
@@ -1513,76 +1515,123 @@ static int mlp_batch_bufs(mlcp_mlp* q, int nb) {
   if (q->X0.need((size_t)nb * m.nx()) || q->Z1.need((size_t)nb * m.nhid) ||
       q->Z2.need((size_t)nb * m.nhid) || q->Y.need((size_t)nb * m.nout) ||
       q->dY.need((size_t)nb * m.nout) || q->dH2.need((size_t)nb * m.nhid) ||
-      q->dH1.need((size_t)nb * m.nhid) || q->dX0.need((size_t)nb * m.nx()))
+      q->dH1.need((size_t)nb * m.nhid) || q->dXe.need((size_t)nb * m.nemb))
     return -1;
   q->nbmax = nb;
   return 0;
 }
 
-static void mlp_gemm(hipStream_t st, int M, int N, int K, const float* A,
-                     long ai, long ak, const float* B, long bj, long bk,
-                     float* C, long ldc, const float* bias, int act, int acc) {
-  dim3 grid((N + MLP_T - 1) / MLP_T, (M + MLP_T - 1) / MLP_T);
-  hipLaunchKernelGGL(k_mlp_gemm, grid, dim3(MLP_T * MLP_T), 0, st, M, N, K,
-                     A, ai, ak, B, bj, bk, C, ldc, bias, act, acc);
+template <int KFB>
+static void mlp_gemm(hipStream_t st, MlpOp A, MlpOp B, int K, MlpOut o) {
+  dim3 grid((B.n + MLP_TJ - 1) / MLP_TJ, (A.n + MLP_TI - 1) / MLP_TI);
+  hipLaunchKernelGGL(k_mlp_gemm<KFB>, grid, dim3(256), 0, st, A, B, K, o);
 }
 
 // Forward pass of nb rows (X0 already gathered) on stream st:
 // Z1 = tanh(X0 W1^T + b1), Z2 = tanh(Z1 W2^T + b2), Y = x + Z2 W3^T + b3
-// (Z1, Z2 hold the activations).
-static void mlp_forward_rows(mlcp_mlp* q, int nb, hipStream_t st) {
+// (Z1, Z2 hold the activations).  With a target (T, by idx) the output layer
+// leaves dY and the squared error instead of Y.
+static void mlp_forward_rows(mlcp_mlp* q, int nb, hipStream_t st,
+                             const float* T = nullptr,
+                             const int* idx = nullptr) {
   const MlpDims& m = q->m;
   const float* P = q->P.p;
-  mlp_gemm(st, nb, m.nhid, m.nx(), q->X0.p, m.nx(), 1, P + m.oW1(), m.nx(),
-           1, q->Z1.p, m.nhid, P + m.ob1(), 1, 0);
-  mlp_gemm(st, nb, m.nhid, m.nhid, q->Z1.p, m.nhid, 1, P + m.oW2(),
-           m.nhid, 1, q->Z2.p, m.nhid, P + m.ob2(), 1, 0);
-  hipLaunchKernelGGL(k_mlp_skip, dim3(256), dim3(256), 0, st, nb, m.nout,
-                     m.nx(), (const float*)q->X0.p, q->Y.p);
-  mlp_gemm(st, nb, m.nout, m.nhid, q->Z2.p, m.nhid, 1, P + m.oW3(),
-           m.nhid, 1, q->Y.p, m.nout, P + m.ob3(), 0, 1);
+  MlpOut o{};
+  o.C = q->Z1.p;
+  o.ldc = m.nhid;
+  o.bias = P + m.ob1();
+  o.tanh = 1;
+  mlp_gemm<1>(st, {q->X0.p, m.nx(), nb}, {P + m.oW1(), m.nx(), m.nhid},
+           m.nx(), o);
+  o.C = q->Z2.p;
+  o.bias = P + m.ob2();
+  mlp_gemm<1>(st, {q->Z1.p, m.nhid, nb}, {P + m.oW2(), m.nhid, m.nhid},
+           m.nhid, o);
+  o = MlpOut{};
+  o.C = T ? nullptr : q->Y.p;
+  o.ldc = m.nout;
+  o.bias = P + m.ob3();
+  o.skip = q->X0.p;
+  o.lds = m.nx();
+  o.T = T;
+  o.idx = idx;
+  o.scale = 1.0f / nb;
+  o.dY = q->dY.p;
+  o.sse = q->sse.p;
+  mlp_gemm<1>(st, {q->Z2.p, m.nhid, nb}, {P + m.oW3(), m.nhid, m.nout},
+           m.nhid, o);
 }
 
 // Loss and gradient (into G) of nb rows idx[] of the set (X, modes, T).
 static int mlp_loss_grad_rows(mlcp_mlp* q, const float* X, const int* modes,
                               const float* T, const int* idx, int nb) {
   const MlpDims& m = q->m;
-  if (mlp_batch_bufs(q, nb) || q->sse.need(1)) return -1;
-  hipLaunchKernelGGL(k_mlp_input, dim3(256), dim3(256), 0, q->st, m, X, modes,
-                     idx, nb, q->P.p, q->X0.p);
-  mlp_forward_rows(q, nb, q->st);
-  hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, q->st, q->sse.p, 1L, 0.0);
-  hipLaunchKernelGGL(k_mlp_dy, dim3(256), dim3(256), 0, q->st, nb, m.nout,
-                     q->Y.p, T, idx, 1.0f / nb, q->dY.p, q->sse.p);
-  float* G = q->G.p;
-  // layer 3: dW3 = dY^T Z2, db3 = sum dY, dH2 = dY W3
-  mlp_gemm(q->st, m.nout, m.nhid, nb, q->dY.p, 1, m.nout, q->Z2.p, 1, m.nhid,
-           G + m.oW3(), m.nhid, nullptr, 0, 0);
-  hipLaunchKernelGGL(k_mlp_colsum, dim3((m.nout + 63) / 64), dim3(64), 0,
-                     q->st, nb, m.nout, q->dY.p, G + m.ob3());
-  mlp_gemm(q->st, nb, m.nhid, m.nout, q->dY.p, m.nout, 1, q->P.p + m.oW3(), 1,
-           m.nhid, q->dH2.p, m.nhid, nullptr, 0, 0);
-  hipLaunchKernelGGL(k_mlp_dtanh, dim3(256), dim3(256), 0, q->st,
-                     (long)nb * m.nhid, q->Z2.p, q->dH2.p);
-  // layer 2
-  mlp_gemm(q->st, m.nhid, m.nhid, nb, q->dH2.p, 1, m.nhid, q->Z1.p, 1, m.nhid,
-           G + m.oW2(), m.nhid, nullptr, 0, 0);
-  hipLaunchKernelGGL(k_mlp_colsum, dim3((m.nhid + 63) / 64), dim3(64), 0,
-                     q->st, nb, m.nhid, q->dH2.p, G + m.ob2());
-  mlp_gemm(q->st, nb, m.nhid, m.nhid, q->dH2.p, m.nhid, 1, q->P.p + m.oW2(),
-           1, m.nhid, q->dH1.p, m.nhid, nullptr, 0, 0);
-  hipLaunchKernelGGL(k_mlp_dtanh, dim3(256), dim3(256), 0, q->st,
-                     (long)nb * m.nhid, q->Z1.p, q->dH1.p);
-  // layer 1 and the embedding
-  mlp_gemm(q->st, m.nhid, m.nx(), nb, q->dH1.p, 1, m.nhid, q->X0.p, 1, m.nx(),
-           G + m.oW1(), m.nx(), nullptr, 0, 0);
-  hipLaunchKernelGGL(k_mlp_colsum, dim3((m.nhid + 63) / 64), dim3(64), 0,
-                     q->st, nb, m.nhid, q->dH1.p, G + m.ob1());
-  mlp_gemm(q->st, nb, m.nx(), m.nhid, q->dH1.p, m.nhid, 1, q->P.p + m.oW1(),
-           1, m.nx(), q->dX0.p, m.nx(), nullptr, 0, 0);
-  hipLaunchKernelGGL(k_mlp_embgrad, dim3((m.nmodes * m.nemb + 63) / 64),
-                     dim3(64), 0, q->st, m, nb, modes, idx, q->dX0.p,
-                     G + m.oE());
+  // the gradients' parts: row ranges of at least 128 until the tiles make
+  // three workgroups a CU (4096 rows of 60 inputs: 32 parts of 21 workgroups)
+  MlpGrad g{};
+  int nt = 0;
+  const int gi[3] = {m.nhid, m.nhid, m.nout}, gj[3] = {m.nx(), m.nhid, m.nhid};
+  for (int l = 0; l < 3; l++) {
+    g.t0[l] = nt;
+    nt += ((gi[l] + MLP_TI - 1) / MLP_TI) * ((gj[l] + MLP_TJ - 1) / MLP_TJ);
+  }
+  g.t0[3] = nt;
+  const int want = std::max(1, 3 * q->cus / nt);
+  g.kc = std::max(128, ((nb + want - 1) / want + 63) / 64 * 64);
+  const int ns = (nb + g.kc - 1) / g.kc;
+  if (mlp_batch_bufs(q, nb) || q->sse.need(1) ||
+      q->part.need((size_t)ns * m.np()))
+    return -1;
+  hipStream_t st = q->st;
+  const float* P = q->P.p;
+  hipLaunchKernelGGL(k_mlp_input, dim3(256), dim3(256), 0, st, m, X, modes,
+                     idx, nb, P, q->X0.p, q->sse.p);
+  mlp_forward_rows(q, nb, st, T, idx);
+  // back through the layers: dH2 = (dY W3) (1 - Z2^2), dH1 = (dH2 W2)
+  // (1 - Z1^2), and of the input's gradient the embedding's columns
+  MlpOut o{};
+  o.C = q->dH2.p;
+  o.ldc = m.nhid;
+  o.H = q->Z2.p;
+  mlp_gemm<0>(st, {q->dY.p, m.nout, nb}, {P + m.oW3(), m.nhid, m.nhid},
+           m.nout, o);
+  o.C = q->dH1.p;
+  o.H = q->Z1.p;
+  mlp_gemm<0>(st, {q->dH2.p, m.nhid, nb}, {P + m.oW2(), m.nhid, m.nhid},
+           m.nhid, o);
+  if (m.nemb > 0) {
+    o.C = q->dXe.p;
+    o.ldc = m.nemb;
+    o.H = nullptr;
+    mlp_gemm<0>(st, {q->dH1.p, m.nhid, nb},
+             {P + m.oW1() + m.nin, m.nx(), m.nemb}, m.nhid, o);
+  }
+  g.A[0] = {q->dH1.p, m.nhid, m.nhid};
+  g.B[0] = {q->X0.p, m.nx(), m.nx()};
+  g.A[1] = {q->dH2.p, m.nhid, m.nhid};
+  g.B[1] = {q->Z1.p, m.nhid, m.nhid};
+  g.A[2] = {q->dY.p, m.nout, m.nout};
+  g.B[2] = {q->Z2.p, m.nhid, m.nhid};
+  g.oW[0] = m.oW1();
+  g.oW[1] = m.oW2();
+  g.oW[2] = m.oW3();
+  g.ob[0] = m.ob1();
+  g.ob[1] = m.ob2();
+  g.ob[2] = m.ob3();
+  g.nb = nb;
+  g.dXe = q->dXe.p;
+  g.modes = modes;
+  g.idx = idx;
+  g.nemb = m.nemb;
+  g.nmodes = m.nmodes;
+  g.oE = m.oE();
+  g.np = m.np();
+  g.part = q->part.p;
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nt + (m.nemb > 0 ? 1 : 0), ns),
+                     dim3(256), 0, st, g);
+  hipLaunchKernelGGL(k_mlp_gsum, dim3((unsigned)((m.np() + 255) / 256)),
+                     dim3(256), 0, st, m.np(), ns, (const float*)q->part.p,
+                     q->G.p);
   HCHK(hipGetLastError());
   return 0;
 }
@@ -1597,7 +1646,11 @@ extern "C" int mlcp_mlp_create(mlcp_mlp** out, int nin, int nemb, int nmodes,
   mlcp_mlp* q = new mlcp_mlp();
   q->m = {nin, nemb, nmodes, nhid, nin};
   const long np = q->m.np();
-  if (hipStreamCreateWithFlags(&q->st, hipStreamNonBlocking) != hipSuccess) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&q->cus, hipDeviceAttributeMultiprocessorCount,
+                            dev) != hipSuccess ||
+      hipStreamCreateWithFlags(&q->st, hipStreamNonBlocking) != hipSuccess) {
     delete q;
     return fail("hipStreamCreate failed");
   }
@@ -1709,7 +1762,7 @@ extern "C" int mlcp_mlp_forward(mlcp_mlp* q, const float* X, const int* modes,
     return -1;
   hipLaunchKernelGGL(k_mlp_input, dim3(256), dim3(256), 0, q->st, q->m,
                      q->tX.p, q->tM.p, (const int*)nullptr, N, q->P.p,
-                     q->X0.p);
+                     q->X0.p, (double*)nullptr);
   mlp_forward_rows(q, N, q->st);
   HCHK(hipMemcpyAsync(Y, q->Y.p, sizeof(float) * N * q->m.nout,
                       hipMemcpyDeviceToHost, q->st));
@@ -1782,7 +1835,8 @@ static int mlp_warm_start(mlcp_session* s, int c0, int ncol) {
   hipLaunchKernelGGL(k_ws_gather, dim3(256), dim3(256), 0, s->st, s->pool, c0,
                      ncol, m.nin, q->wX.p, q->wM.p);
   hipLaunchKernelGGL(k_mlp_input, dim3(256), dim3(256), 0, s->st, m, q->wX.p,
-                     q->wM.p, (const int*)nullptr, rows, q->P.p, q->X0.p);
+                     q->wM.p, (const int*)nullptr, rows, q->P.p, q->X0.p,
+                     (double*)nullptr);
   mlp_forward_rows(q, rows, s->st);
   hipLaunchKernelGGL(k_ws_scatter, dim3(256), dim3(256), 0, s->st, s->pool,
                      c0, ncol, m.nout, (const float*)q->Y.p);
