@@ -2639,89 +2639,168 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
 // primitive operators of a mode, Updater.f90:53-107, each through
 // UpdateOperMat, :109-153): QXQ_o(i,j) = <Q_j, X_o Q_i>, i <= j.
 
-// Y_o(:, c) = X_o q_c^{d_o} for every column c of the block (X_o dense, row
-// major, n x n at xoff[o]; Y_o column major n x ncol at yoff[o]).  Operator
-// o is blockIdx.y.
-__global__ void k_opx_apply(Pool p, int ncol, const int* opmode,
-                            const double* X, const long* xoff, double* Y,
-                            const long* yoff) {
-  const int o = blockIdx.y;
-  const int d = opmode[o], n = p.nbas[d];
-  const double* x = X + xoff[o];
-  double* y = Y + yoff[o];
-  const long tot = (long)ncol * n;
+// With the pair's density on the operator's mode,
+//   Z_ij(l, m) = sum_{r in i, s in j} c_r c_s q_r(l) q_s(m)
+//                prod_{d != d_o} <q_r^d, q_s^d>,
+// every operator of the mode is one sum QXQ_o(i,j) = sum_{l,m} X_o(l, m)
+// Z_ij(l, m): R^2 n + R n^2 multiplications a pair and mode and n^2 an
+// operator, instead of R^2 n an operator.
+
+// Block of the operator update: the factors of mode d as columns of NP =
+// 16 ceil(n/16) doubles, zero past n, at q + off[d].
+struct OpxBlock {
+  int ndof;
+  int nbas[MLCP_MAXD];
+  int nt[MLCP_MAXD];     // tiles of 16 rows
+  long off[MLCP_MAXD];
+  int op0[MLCP_MAXD + 1];   // the operators of each mode in ops
+  double* q;
+  const double* coef;
+  int ncol;
+};
+
+// The modes of one launch.
+struct OpxModes {
+  int d[MLCP_MAXD];
+};
+
+// Fills the block's mode blockIdx.y from the column-by-column input.
+__global__ void k_opx_pack(OpxBlock b, const double* in) {
+  const int d = blockIdx.y, n = b.nbas[d], np = 16 * b.nt[d];
+  int row0 = 0, nD = 0;
+  for (int e = 0; e < b.ndof; e++) {
+    if (e < d) row0 += b.nbas[e];
+    nD += b.nbas[e];
+  }
+  double* q = b.q + b.off[d];
+  const long tot = (long)b.ncol * np;
   for (long e = blockIdx.x * (long)blockDim.x + TID; e < tot;
        e += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(e / n), m = (int)(e % n);
-    const double* q = colp(p, d, c);
-    double s = 0.0;
-    for (int l = 0; l < n; l++) s = fma(x[(long)m * n + l], q[l], s);
-    y[e] = s;
+    const long c = e / np;
+    const int m = (int)(e - c * np);
+    q[e] = m < n ? in[c * nD + row0 + m] : 0.0;
   }
 }
 
-#define OPX_G 16   // operators per pass of k_opx_pairs
-
-// One workgroup per state pair (i, j), i <= j:
-//   out[o*npk + i + j(j+1)/2] = sum_{r in i, s in j} c_r c_s
-//       <q_s^{d_o}, X_o q_r^{d_o}> prod_{d != d_o} <q_r^d, q_s^d>
-// for every operator o.  The per-mode Grams of a term pair (r, s) are formed
-// once per pass of OPX_G operators and kept in LDS; each thread sums its
-// term pairs in a fixed order, then the workgroup reduces (wave shuffles,
-// then the four waves in order), so the result does not depend on timing.
-__global__ __launch_bounds__(MLCP_NT) void k_opx_pairs(
-    Pool p, const int* roff, const int* ranks, const int2* pairs, int nops,
-    const int* opmode, const double* Y, const long* yoff, double* out,
-    long npk) {
-  __shared__ double gsh[MLCP_MAXD][MLCP_NT];
-  __shared__ double wsum[OPX_G][MLCP_NT / 64];
-  const int2 pr = pairs[blockIdx.x];
+// Densities and operators of mode d (blockIdx.y), a wave per state pair (i, j) and
+// group of LG row tiles of the density (NG = ceil(NT / LG) waves share a pair
+// where the NT x NT tiles exceed a wave's registers).  Everything stays in the
+// matrix-core layouts: the transposed Gram tile (s, r) is, register by
+// register, the A operand of T(r, m) = sum_s E(r, s) q_s(m), whose tiles are
+// in turn the B operand of Z(l, m) += sum_r q_r(l) T(r, m), so there is
+// neither LDS nor a shuffle before the final sums.  Bound by the FP64 matrix
+// rate and the L1 reads of the operands and of X: 120 states of rank 10-30,
+// 28 operators on two modes of 40: 385 us (dot products of strided
+// columns, operator by operator: 5.1 ms), half of them for the operators.
+template <int NT, int LG>
+__global__ __launch_bounds__(256) void k_opx_density(
+    OpxBlock b, OpxModes ms, const int* roff, const int* ranks,
+    const int2* pairs, int npairs, const int* opl, const double* X,
+    const long* xoff, double* out, long npk) {
+  constexpr int NG = (NT + LG - 1) / LG, NP = 16 * NT, U = 4;
+  __shared__ double ws[4][U];
+  const int lane = TID & 63, lr = lane & 15, lq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(TID >> 6);
+  const int g = w % NG, l0 = g * LG, d = ms.d[blockIdx.y];
+  const int* ops = opl + b.op0[d];
+  const int nops = b.op0[d + 1] - b.op0[d];
+  const int u0 = blockIdx.x * (4 / NG) + w / NG;
+  const int2 pr = pairs[min(u0, npairs - 1)];
   const int i = pr.x, j = pr.y;
   const int Ri = ranks[i], Rj = ranks[j], ci = roff[i], cj = roff[j];
-  const int D = p.ndof;
-  const int lane = TID & 63, w = TID >> 6;
-  for (int o0 = 0; o0 < nops; o0 += OPX_G) {
-    double acc[OPX_G];
+  const v4d zero = {0.0, 0.0, 0.0, 0.0};
+  const double* q = b.q + b.off[d];
+  v4d Z[LG][NT];
 #pragma unroll
-    for (int u = 0; u < OPX_G; u++) acc[u] = 0.0;
-    for (int e = TID; e < Ri * Rj; e += MLCP_NT) {
-      const int r = e / Rj, s = e - r * Rj;
-      for (int d = 0; d < D; d++) {
-        const double* a = colp(p, d, ci + r);
-        const double* b = colp(p, d, cj + s);
-        double g = 0.0;
-        for (int m = 0; m < p.nbas[d]; m++) g = fma(a[m], b[m], g);
-        gsh[d][TID] = g;
+  for (int lt = 0; lt < LG; lt++)
+#pragma unroll
+    for (int mt = 0; mt < NT; mt++) Z[lt][mt] = zero;
+  for (int r0 = 0; r0 < Ri; r0 += 16) {
+    const int rr = ci + min(r0 + lr, Ri - 1);
+    const double cr = ld_or0(b.coef + rr, r0 + lr < Ri);
+    v4d T[NT];
+#pragma unroll
+    for (int mt = 0; mt < NT; mt++) T[mt] = zero;
+    for (int s0 = 0; s0 < Rj; s0 += 16) {
+      // E(s, r) = c_r c_s prod of the other modes' Grams: register v of lane
+      // (lq, lr) is s = s0 + lq + 4 v, r = r0 + lr; zero past the ranks
+      v4d E;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int s = s0 + lq + 4 * v;
+        E[v] = cr * ld_or0(b.coef + cj + min(s, Rj - 1), s < Rj);
       }
-      const double wgt = p.coef[ci + r] * p.coef[cj + s];
+      for (int dd = 0; dd < b.ndof; dd++) {
+        if (dd == d) continue;
+        const int np = 16 * b.nt[dd];
+        const double* pa = b.q + b.off[dd] + (long)(cj + min(s0 + lr, Rj - 1)) * np + lq;
+        const double* pb = b.q + b.off[dd] + (long)rr * np + lq;
+        v4d G = zero;
+        for (int k = 0; k < np; k += 16)
 #pragma unroll
-      for (int u = 0; u < OPX_G; u++) {
-        const int o = o0 + u;
-        if (o < nops) {
-          const int d = opmode[o], n = p.nbas[d];
-          const double* yr = Y + yoff[o] + (long)(ci + r) * n;
-          const double* qs = colp(p, d, cj + s);
-          double t = 0.0;
-          for (int m = 0; m < n; m++) t = fma(qs[m], yr[m], t);
-          double ex = 1.0;
-          for (int dd = 0; dd < D; dd++)
-            if (dd != d) ex *= gsh[dd][TID];
-          acc[u] += wgt * ex * t;
+          for (int x = 0; x < 16; x += 4) G = mfma_f64_4(pa[k + x], pb[k + x], G);
+        E *= G;
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const double* pb = q + (long)(cj + min(s0 + 4 * v + lq, Rj - 1)) * NP + lr;
+#pragma unroll
+        for (int mt = 0; mt < NT; mt++) T[mt] = mfma_f64_4(E[v], pb[16 * mt], T[mt]);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const double* pa = q + (long)(ci + min(r0 + 4 * v + lq, Ri - 1)) * NP + lr;
+#pragma unroll
+      for (int lt = 0; lt < LG; lt++) {
+        const double a = pa[16 * min(l0 + lt, NT - 1)];
+#pragma unroll
+        for (int mt = 0; mt < NT; mt++) Z[lt][mt] = mfma_f64_4(a, T[mt][v], Z[lt][mt]);
+      }
+    }
+  }
+  // the operators, U at a time: lane (lq, lr) holds Z(l, m) for l = 16 lt +
+  // lq + 4 v, m = 16 mt + lr
+  const long at = i + (long)j * (j + 1) / 2;
+  for (int o0 = 0; o0 < nops; o0 += U) {
+    double sum[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const double* x = X + xoff[ops[min(o0 + u, nops - 1)]] + lq * NP + lr;
+      double t = 0.0;
+#pragma unroll
+      for (int lt = 0; lt < LG; lt++) {
+        if (LG * NG == NT || l0 + lt < NT) {   // uniform
+#pragma unroll
+          for (int mt = 0; mt < NT; mt++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+              t = fma(Z[lt][mt][v], x[(16 * (l0 + lt) + 4 * v) * NP + 16 * mt], t);
         }
       }
+      sum[u] = t;
     }
 #pragma unroll
-    for (int u = 0; u < OPX_G; u++) {
-      double v = acc[u];
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-      if (lane == 0) wsum[u][w] = v;
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int u = 0; u < U; u++) sum[u] += __shfl_xor(sum[u], o, 64);
+    if constexpr (NG == 1) {
+      if (lane == 0 && u0 < npairs)
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (o0 + u < nops) out[(long)ops[o0 + u] * npk + at] = sum[u];
+    } else {
+      if (lane == 0)
+#pragma unroll
+        for (int u = 0; u < U; u++) ws[w][u] = sum[u];
+      __syncthreads();
+      if (g == 0 && lane < U && u0 < npairs && o0 + lane < nops) {
+        double t = 0.0;
+#pragma unroll
+        for (int x = 0; x < NG; x++) t += ws[w + x][lane];
+        out[(long)ops[o0 + lane] * npk + at] = t;
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    if (TID < OPX_G && o0 + TID < nops) {
-      double v = 0.0;
-      for (int q = 0; q < MLCP_NT / 64; q++) v += wsum[TID][q];
-      out[(long)(o0 + TID) * npk + i + (long)j * (j + 1) / 2] = v;
-    }
-    __syncthreads();
   }
 }

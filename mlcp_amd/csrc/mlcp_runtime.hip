@@ -2381,29 +2381,34 @@ extern "C" int mlcp_hip_update_opers(const double* base, const double* coef,
     roff[s] = Ntot;
     Ntot += ranks[s];
   }
-  // dense operators (row major) and the offsets of their Y blocks
-  std::vector<int> om(nops);
-  std::vector<long> xoff(nops), yoff(nops);
+  // dense operators, padded with zeros to whole tiles, and the operators of
+  // each mode
+  std::vector<std::vector<int>> mops(ndof);
+  std::vector<long> xoff(nops);
   std::vector<double> X;
-  long ytot = 0;
   for (int o = 0; o < nops; o++) {
     if (opmode[o] < 1 || opmode[o] > ndof)
       return fail("opmode must be in 1..ndof");
-    const int d = opmode[o] - 1, n = nbas[d];
+    const int d = opmode[o] - 1, n = nbas[d], np = (n + 15) / 16 * 16;
     const long nq = (long)n * (n + 1) / 2;
     if (mptr[o] < 1 || mptr[o] - 1 + nq > msize)
       return fail("operator " + std::to_string(o) + " exceeds mat");
     const double* ap = mat + (mptr[o] - 1);
-    om[o] = d;
+    mops[d].push_back(o);
     xoff[o] = (long)X.size();
-    yoff[o] = ytot;
-    ytot += (long)n * Ntot;
-    for (int a = 0; a < n; a++)
-      for (int b = 0; b < n; b++) {
-        const int lo = std::min(a, b), hi = std::max(a, b);
-        X.push_back(ap[lo + (long)hi * (hi + 1) / 2]);
-      }
+    X.resize(X.size() + (size_t)np * np, 0.0);
+    double* x = X.data() + xoff[o];
+    for (int hi = 0; hi < n; hi++)
+      for (int lo = 0; lo <= hi; lo++)
+        x[lo * np + hi] = x[hi * np + lo] = *ap++;
   }
+  OpxBlock blk{};
+  std::vector<int> om;   // operators by mode
+  for (int d = 0; d < ndof; d++) {
+    blk.op0[d] = (int)om.size();
+    om.insert(om.end(), mops[d].begin(), mops[d].end());
+  }
+  blk.op0[ndof] = nops;
   std::vector<int2> pairs;
   for (int j = 0; j < nbloc; j++)
     for (int i = 0; i <= j; i++) pairs.push_back(make_int2(i, j));
@@ -2414,43 +2419,56 @@ extern "C" int mlcp_hip_update_opers(const double* base, const double* coef,
     hipStream_t s;
     ~StreamGuard() { (void)hipStreamDestroy(s); }
   } sg{st};
-  DBuf<double> fac, cf, stage, dX, dY, dout;
+  blk.ndof = ndof;
+  blk.ncol = Ntot;
+  size_t qtot = 0;
+  for (int d = 0; d < ndof; d++) {
+    blk.nbas[d] = nbas[d];
+    blk.nt[d] = (nbas[d] + 15) / 16;
+    blk.off[d] = (long)qtot;
+    qtot += (size_t)16 * blk.nt[d] * Ntot;
+  }
+  const size_t nb = (size_t)nD * Ntot;
+  DBuf<double> q, cf, stage, dX, dout;
   DBuf<int> dR, dro, dom;
-  DBuf<long> dxo, dyo;
+  DBuf<long> dxo;
   DBuf<int2> dpairs;
-  if (fac.need((size_t)nD * Ntot) || cf.need(Ntot) ||
-      stage.need((size_t)nD * Ntot + Ntot) || dX.put(X, st) ||
-      dY.need((size_t)ytot) || dout.need((size_t)nops * npk) ||
+  if (q.need(qtot) || cf.need(Ntot) || stage.need(nb) || dX.put(X, st) ||
+      dout.need((size_t)nops * npk) ||
       dR.put(std::vector<int>(ranks, ranks + nbloc), st) ||
       dro.put(roff, st) || dom.put(om, st) || dxo.put(xoff, st) ||
-      dyo.put(yoff, st) || dpairs.put(pairs, st))
+      dpairs.put(pairs, st))
     return -1;
-  Pool pool;
-  pool.ndof = ndof;
-  long off = 0;
-  for (int d = 0; d < ndof; d++) {
-    pool.nbas[d] = nbas[d];
-    pool.moff[d] = off;
-    off += (long)nbas[d] * Ntot;
-  }
-  pool.fac = fac.p;
-  pool.coef = cf.p;
-  const size_t nb = (size_t)nD * Ntot;
+  blk.q = q.p;
+  blk.coef = cf.p;
   HCHK(hipMemcpyAsync(stage.p, base, nb * sizeof(double),
                       hipMemcpyHostToDevice, st));
-  HCHK(hipMemcpyAsync(stage.p + nb, coef, Ntot * sizeof(double),
+  HCHK(hipMemcpyAsync(cf.p, coef, Ntot * sizeof(double),
                       hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_to_pool, dim3(512), dim3(256), 0, st, stage.p,
-                     stage.p + nb, pool, 0, Ntot, nD);
-  const long napply = (long)Ntot * nmax;
-  hipLaunchKernelGGL(k_opx_apply,
-                     dim3((unsigned)std::min<long>(1024, (napply + 255) / 256),
-                          nops),
-                     dim3(256), 0, st, pool, Ntot, dom.p, dX.p, dxo.p, dY.p,
-                     dyo.p);
-  hipLaunchKernelGGL(k_opx_pairs, dim3((unsigned)pairs.size()), dim3(MLCP_NT),
-                     0, st, pool, dro.p, dR.p, dpairs.p, nops, dom.p, dY.p,
-                     dyo.p, dout.p, npk);
+  hipLaunchKernelGGL(k_opx_pack, dim3(64, ndof), dim3(256), 0, st, blk,
+                     (const double*)stage.p);
+  // one launch for all modes of as many tiles
+  const int npairs = (int)pairs.size();
+  for (int nt = 1; nt <= MLCP_NMAX / 16; nt++) {
+    OpxModes ms{};
+    int nm = 0;
+    for (int d = 0; d < ndof; d++)
+      if (blk.nt[d] == nt && !mops[d].empty()) ms.d[nm++] = d;
+    if (!nm) continue;
+#define OPX(NT, LG)                                                          \
+  case NT: {                                                                 \
+    constexpr int per = 4 / ((NT + LG - 1) / LG); /* pairs a workgroup */    \
+    hipLaunchKernelGGL((k_opx_density<NT, LG>),                              \
+                       dim3((npairs + per - 1) / per, nm), dim3(256), 0, st, \
+                       blk, ms, dro.p, dR.p, dpairs.p, npairs, dom.p,        \
+                       (const double*)dX.p, dxo.p, dout.p, npk);             \
+  } break;
+    switch (nt) {
+      OPX(1, 1) OPX(2, 2) OPX(3, 3) OPX(4, 4)
+      OPX(5, 3) OPX(6, 3) OPX(7, 2) OPX(8, 2)
+    }
+#undef OPX
+  }
   HCHK(hipGetLastError());
   HCHK(hipMemcpyAsync(out, dout.p, (size_t)nops * npk * sizeof(double),
                       hipMemcpyDeviceToHost, st));
