@@ -2183,7 +2183,13 @@ __global__ __launch_bounds__(MLCP_NT) void k_pair_inner(Pool p,
 // Every step of 1-3 and 5 touches O(n^2) entries between two barriers (O(n)
 // steps, O(n^3) work); 4 is a chain of about n^2 dependent rotations, two
 // sweeps per eigenvalue on average.  MODE 1
-// keeps the working matrix in LDS (dynamic: n*(n|1) doubles), MODE 0 in ws.
+// keeps the working matrix in LDS (dynamic: n*(n|1) doubles) and does
+// everything (PART 0).  Larger matrices (MODE 0, from n = 132 on) stay in ws,
+// where one workgroup's sweeps wait for L2; of them only what is one chain
+// runs here (PART 2: steps 3 and 4, the rotations applied to the identity);
+// k_gep_chol does step 1 in registers, k_gep_subst and k_gep_back steps 2 and
+// 5 and the application of Q on all CUs.  n = 200: 6.6 ms,
+// 19.5 ms in one workgroup.
 // ws: U (n*n), then the working matrix (n*n, MODE 0).  Output X column major
 // n x n into Xo, w into wo.  Error bits (outputs untouched): 4 S not
 // positive definite, 8 non-finite entries or no QL convergence.
@@ -2193,7 +2199,7 @@ __global__ __launch_bounds__(MLCP_NT) void k_pair_inner(Pool p,
 // 256, the fewest that hold m) and GEP_NT >> gep_sh(m) column phases, so a
 // small trailing block still spreads over every thread.
 __device__ __forceinline__ int gep_sh(int m) { return m <= 64 ? 6 : (m <= 128 ? 7 : 8); }
-template <int MODE>
+template <int MODE, int PART>
 __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
                                                 const double* Sin, int n,
                                                 double* ws, double* Xo,
@@ -2202,18 +2208,27 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
   __shared__ double s_u[2][MLCP_BMAX];     // staged row/column of U
   __shared__ double s_v[2][MLCP_BMAX];     // Householder vector x of a step
   __shared__ double s_p[MLCP_BMAX];        // p = b C v, then y = b v^T Q
-  __shared__ double s_d[MLCP_BMAX], s_e[MLCP_BMAX], s_b[MLCP_BMAX];
-  __shared__ double s_rc[2][MLCP_BMAX], s_rs[2][MLCP_BMAX];
+  // subdiagonal and diagonal side by side, eight entries of room before the
+  // first (reads ahead of the chain need no clamp); rotations likewise
+  __shared__ __align__(16) double2 s_ed[MLCP_BMAX + 8];
+  __shared__ __align__(16) double2 s_cs[2][MLCP_BMAX];
+  __shared__ double s_b[MLCP_BMAX];
   __shared__ double s_part[2][GEP_NT / 64], s_q[GEP_NT / 64];
   __shared__ int s_lohi[2][2];
   __shared__ int s_flag[2];
   __shared__ int s_ord[MLCP_BMAX];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ld = MODE == 1 ? (n | 1) : n;
   double* U = ws;
   double* M = MODE == 1 ? gsh : ws + (long)n * n;
 #define GM(i, j) M[(i) + (long)(j) * ld]
 #define GU(i, j) U[(i) + (long)(j) * n]
+#define SE(i) s_ed[8 + (i)].x
+#define SD(i) s_ed[8 + (i)].y
+  if constexpr (PART == 2) {
+    if (*err & 12) return;   // an earlier part failed
+  } else {
   // ---- 1. Cholesky: S (upper triangle) -> M, full symmetric
   for (int e = tid; e < n * n; e += GEP_NT) {
     const int i = e % n, j = e / n;
@@ -2291,6 +2306,7 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
     GM(i, j) /= GU(i, i);
   }
   __syncthreads();
+  }
   for (int e = tid; e < n * n; e += GEP_NT) {
     const int i = e % n, j = e / n;
     if (i < j) {
@@ -2327,16 +2343,29 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
     const double v0 = sig == 0.0 ? x0 : (x0 <= 0.0 ? x0 - mu : x0 + mu);
     const double b = sig == 0.0 ? 0.0 : 2.0 / (v0 * v0 + sig);
     if (tid == 0) {
-      s_d[k] = GM(k, k);
+      SD(k) = GM(k, k);
       s_b[k] = b;
-      s_e[k] = sig == 0.0 ? x0 : (x0 <= 0.0 ? mu : -mu);
+      SE(k) = sig == 0.0 ? x0 : (x0 <= 0.0 ? mu : -mu);
       GM(k + 1, k) = v0;   // column k keeps v for the forming of Q
     }
     // p = b B v: 2^tsh threads per row (adjacent lanes), shuffled together
     {
       const int r = tid >> tsh, tq = tid & ((1 << tsh) - 1), ts = 1 << tsh;
       double s = 0.0, s2 = 0.0;
-      if (r < m) {
+      if constexpr (MODE == 0) {
+        if (r < m)
+          for (int c0 = tq; c0 < m; c0 += 8 * ts) {
+            double a[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+              a[u] = GM(k + 1 + r, k + 1 + min(c0 + u * ts, m - 1));
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+              const int c = c0 + u * ts;
+              if (c < m) s += a[u] * (c == 0 ? v0 : s_v[cb][c]);
+            }
+          }
+      } else if (r < m) {
         int c = tq;
         for (; c + ts < m; c += 2 * ts) {
           s += GM(k + 1 + r, k + 1 + c) * (c == 0 ? v0 : s_v[cb][c]);
@@ -2367,14 +2396,27 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
       if (R < m) {
         const double vr = R == 0 ? v0 : s_v[cb][R];
         const double wr = s_p[R] - K * vr;
-        for (int c = CQ; c < m; c += CP) {
+        if constexpr (PART == 2) {
+          // sqrt(b) v, for the back-transformation
+          if (CQ == 0) GU(k + 1 + R, k) = sqrt(b) * vr;
+        }
+        constexpr int NB = MODE == 0 ? 8 : 1;
+        for (int c0 = CQ; c0 < m; c0 += NB * CP) {
+         double old[NB];
+#pragma unroll
+         for (int u = 0; u < NB; u++)
+           old[u] = GM(k + 1 + R, k + 1 + min(c0 + u * CP, m - 1));
+#pragma unroll
+         for (int u = 0; u < NB; u++) {
+          const int c = c0 + u * CP;
+          if (MODE == 0 && c >= m) continue;
           const double vc = c == 0 ? v0 : s_v[cb][c];
           const double wc = s_p[c] - K * vc;
           double nv;
           {
 #pragma clang fp contract(off)
             const double t = vr * wc + wr * vc;
-            nv = GM(k + 1 + R, k + 1 + c) - t;
+            nv = old[u] - t;
           }
           GM(k + 1 + R, k + 1 + c) = nv;
           // column k+1 below the next diagonal: the next step's x
@@ -2382,6 +2424,7 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
             s_v[nb][R - 1] = nv;
             if (R >= 2) sq = nv * nv;
           }
+         }
         }
       }
       for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
@@ -2391,14 +2434,19 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
   }
   if (tid == 0) {
     if (n >= 2) {
-      s_d[n - 2] = GM(n - 2, n - 2);
-      s_e[n - 2] = GM(n - 1, n - 2);
+      SD(n - 2) = GM(n - 2, n - 2);
+      SE(n - 2) = GM(n - 1, n - 2);
     }
-    s_d[n - 1] = GM(n - 1, n - 1);
-    s_e[n - 1] = 0.0;
+    SD(n - 1) = GM(n - 1, n - 1);
+    SE(n - 1) = 0.0;
     GM(n - 1, n - 1) = 1.0;
   }
   __syncthreads();
+  if constexpr (PART == 2) {
+    // the rotations start from the identity; k_gep_back applies Q
+    for (int e = tid; e < n * n; e += GEP_NT)
+      M[e] = e % n == e / n ? 1.0 : 0.0;
+  } else {
   // Q = H_0 H_1 ... H_{n-3}, formed from the last reflection back: before
   // step k the block (k+2.., k+2..) holds H_{k+1} ... H_{n-3}; row and
   // column k+1 become e_{k+1} (column k+1 below the diagonal held v_{k+1},
@@ -2440,8 +2488,9 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
     GM(i, 0) = 0.0;
     GM(0, i) = 0.0;
   }
+  if (tid == 0) GM(0, 0) = 1.0;
+  }
   if (tid == 0) {
-    GM(0, 0) = 1.0;
     s_flag[0] = 0;
     s_flag[1] = 0;
   }
@@ -2467,8 +2516,8 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
             const int mc = base + lane;
             bool neg = false;
             if (mc < n - 1) {
-              const double dd = fabs(s_d[mc]) + fabs(s_d[mc + 1]);
-              neg = fabs(s_e[mc]) <= 2.220446049250313e-16 * dd;
+              const double dd = fabs(SD(mc)) + fabs(SD(mc + 1));
+              neg = fabs(SE(mc)) <= 2.220446049250313e-16 * dd;
             }
             const unsigned long long bal = __ballot(neg);
             if (bal) {
@@ -2485,62 +2534,120 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
             fin = 2;
             break;
           }
-          const double dl = s_d[l], el = s_e[l];
-          double g = (s_d[l + 1] - dl) / (2.0 * el);
+          const double dl = SD(l), el = SE(l);
+          double g = (SD(l + 1) - dl) / (2.0 * el);
           double r = hypot(g, 1.0);
-          g = s_d[m] - dl + el / (g + (g >= 0.0 ? r : -r));
-          double s = 1.0, c = 1.0, p = 0.0;
-          int i = m - 1;
-          bool under = false;
-          // operands of step i: e(i), d(i), d(i+1), none written before it
-          double ei = s_e[i], di = s_d[i], di1 = s_d[i + 1];
-          for (; i >= l; i--) {
-            const double en = s_e[max(i - 1, 0)], dn = s_d[max(i - 1, 0)];
-            const double f = s * ei, bb = c * ei;
-            const double r2 = f * f + g * g;
-            if (r2 == 0.0) {
-              if (lane == 0) {
-                s_e[i + 1] = 0.0;
-                s_d[i + 1] = di1 - p;
-                s_e[m] = 0.0;
+          g = SD(m) - dl + el / (g + (g >= 0.0 ? r : -r));
+          lo = l;
+          // One lane runs the chain (its stores need no execution mask of
+          // their own), four steps at a time without a branch: d and e come
+          // a block ahead, results stay in registers, and one test at the
+          // end finds the blocks that met anything but positive normal sums
+          // of squares; those are run again step by step.  A step is then
+          // its dozen dependent operations (240 to 270 clocks; 385 with a
+          // test and its branches in every step, 600 with divergent ones).  Products
+          // and sums are written out, not left to contraction.
+          if (lane == 0) {
+#pragma clang fp contract(off)
+            double s = 1.0, c = 1.0, p = 0.0, di1 = SD(m);
+            int i = m - 1;
+            // four steps from i on x, the next four entries to y; false (and
+            // nothing done) if one meets an exception
+            auto block = [&](const double2* x, double2* y)
+                __attribute__((always_inline)) {
+              double2* ed = s_ed + 8 + i - 7;   // ed[7 - q]: entry i - q
+              double2* cs = &s_cs[pb][i - 3];
+              double2 eo[4], co[4];
+#pragma unroll
+              for (int q = 0; q < 4; q++) y[q] = ed[3 - q];
+              double s1 = s, c1 = c, p1 = p, g1 = g, x1 = di1;
+              bool bad = false;
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                const double ei = x[q].x, di = x[q].y;
+                const double f = s1 * ei, bb = c1 * ei;
+                const double r2 = fma(g1, g1, f * f);
+                bad |= !__builtin_amdgcn_class(r2, 0x100);
+                // rsqrt: the hardware's estimate y and one third-order
+                // step, y (1 + h / 2 + 3 h^2 / 8) with h = 1 - r2 y^2
+                const double yy = __builtin_amdgcn_rsq(r2);
+                const double h = fma(-r2 * yy, yy, 1.0);
+                const double ri = fma(yy * h, fma(h, 0.375, 0.5), yy);
+                s1 = f * ri;
+                c1 = g1 * ri;
+                const double gg = x1 - p1;
+                const double qv = fma(di - gg, s1, c1 * (bb + bb));
+                p1 = s1 * qv;
+                eo[q] = make_double2(r2 * ri, gg + p1);
+                co[q] = make_double2(c1, s1);
+                g1 = fma(c1, qv, -bb);
+                x1 = di;
               }
-              under = true;
-              break;
+              // the reads of the next block stay above the steps
+#pragma unroll
+              for (int q = 0; q < 4; q++)
+                asm volatile("" : "+v"(y[q].x), "+v"(y[q].y));
+              if (__builtin_expect(__ballot(bad) != 0, 0)) return false;
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                ed[8 - q] = eo[q];
+                cs[3 - q] = co[q];
+              }
+              s = s1;
+              c = c1;
+              p = p1;
+              g = g1;
+              di1 = x1;
+              i -= 4;
+              return true;
+            };
+            for (;;) {
+              double2 b0[4], b1[4];
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                b0[q] = s_ed[8 + i - q];
+                asm volatile("" : "+v"(b0[q].x), "+v"(b0[q].y));
+              }
+              while (i - 3 >= l) {
+                if (!block(b0, b1)) break;
+                if (i - 3 < l || !block(b1, b0)) break;
+              }
+              if (i < l) break;
+              // one step: of the last three, or of a block with an exception
+              const double ei = SE(i), di = SD(i);
+              const double f = s * ei, bb = c * ei;
+              const double r2 = fma(g, g, f * f);
+              if (__ballot(r2 == 0.0)) break;
+              double rinv;
+              if (__ballot(isfinite(r2))) {
+                rinv = rsqrt(r2);
+                r = r2 * rinv;
+              } else {
+                r = hypot(f, g);
+                rinv = 1.0 / r;
+              }
+              s = f * rinv;
+              c = g * rinv;
+              g = di1 - p;
+              const double qv = fma(di - g, s, c * (bb + bb));
+              p = s * qv;
+              s_ed[8 + i + 1] = make_double2(r, g + p);
+              s_cs[pb][i] = make_double2(c, s);
+              g = fma(c, qv, -bb);
+              di1 = di;
+              if (--i < l) break;
             }
-            double rinv;
-            if (isfinite(r2)) {
-              rinv = rsqrt(r2);
-              r = r2 * rinv;
+            SE(m) = 0.0;
+            if (i >= l) {   // underflow: recover
+              SE(i + 1) = 0.0;
+              SD(i + 1) = di1 - p;
+              lo = i + 1;
             } else {
-              r = hypot(f, g);
-              rinv = 1.0 / r;
+              SD(l) = dl - p;
+              SE(l) = g;
             }
-            s = f * rinv;
-            c = g * rinv;
-            g = di1 - p;
-            const double qv = (di - g) * s + 2.0 * c * bb;
-            p = s * qv;
-            if (lane == 0) {
-              s_e[i + 1] = r;
-              s_d[i + 1] = g + p;
-              s_rc[pb][i] = c;
-              s_rs[pb][i] = s;
-            }
-            g = c * qv - bb;
-            ei = en;
-            di1 = di;
-            di = dn;
           }
-          if (!under) {
-            if (lane == 0) {
-              s_d[l] = dl - p;
-              s_e[l] = g;
-              s_e[m] = 0.0;
-            }
-            lo = l;
-          } else {
-            lo = i + 1;
-          }
+          lo = __builtin_amdgcn_readfirstlane(lo);
           hi = m - 1;
           break;
         }
@@ -2553,26 +2660,25 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
         const int row = tid - 64, ob = pb ^ 1;
         const int lo = s_lohi[ob][0], hi = s_lohi[ob][1];
         if (lo <= hi) {
-          const double* rc = s_rc[ob];
-          const double* rs = s_rs[ob];
+          const double2* cs = s_cs[ob];
           double f = GM(row, hi + 1);
           int i = hi;
           for (; i - 3 >= lo; i -= 4) {
             const double z0 = GM(row, i), z1 = GM(row, i - 1);
             const double z2 = GM(row, i - 2), z3 = GM(row, i - 3);
-            GM(row, i + 1) = rs[i] * z0 + rc[i] * f;
-            f = rc[i] * z0 - rs[i] * f;
-            GM(row, i) = rs[i - 1] * z1 + rc[i - 1] * f;
-            f = rc[i - 1] * z1 - rs[i - 1] * f;
-            GM(row, i - 1) = rs[i - 2] * z2 + rc[i - 2] * f;
-            f = rc[i - 2] * z2 - rs[i - 2] * f;
-            GM(row, i - 2) = rs[i - 3] * z3 + rc[i - 3] * f;
-            f = rc[i - 3] * z3 - rs[i - 3] * f;
+            GM(row, i + 1) = cs[i].y * z0 + cs[i].x * f;
+            f = cs[i].x * z0 - cs[i].y * f;
+            GM(row, i) = cs[i - 1].y * z1 + cs[i - 1].x * f;
+            f = cs[i - 1].x * z1 - cs[i - 1].y * f;
+            GM(row, i - 1) = cs[i - 2].y * z2 + cs[i - 2].x * f;
+            f = cs[i - 2].x * z2 - cs[i - 2].y * f;
+            GM(row, i - 2) = cs[i - 3].y * z3 + cs[i - 3].x * f;
+            f = cs[i - 3].x * z3 - cs[i - 3].y * f;
           }
           for (; i >= lo; i--) {
             const double zi = GM(row, i);
-            GM(row, i + 1) = rs[i] * zi + rc[i] * f;
-            f = rc[i] * zi - rs[i] * f;
+            GM(row, i + 1) = cs[i].y * zi + cs[i].x * f;
+            f = cs[i].x * zi - cs[i].y * f;
           }
           GM(row, lo) = f;
         }
@@ -2582,20 +2688,26 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
     }
   }
   // ---- 5. errors, sort, back-transformation
-  if (tid < n && !isfinite(s_d[tid])) s_flag[1] = 1;
+  if (tid < n && !isfinite(SD(tid))) s_flag[1] = 1;
   __syncthreads();
   if (s_flag[0] != 1 || s_flag[1]) {
     if (tid == 0) atomicOr(err, 8);
     return;
   }
   if (tid < n) {   // rank sort, ties by index
-    const double wi = s_d[tid];
+    const double wi = SD(tid);
     int r = 0;
     for (int j = 0; j < n; j++) {
-      const double wj = s_d[j];
+      const double wj = SD(j);
       if (wj < wi || (wj == wi && j < tid)) r++;
     }
     s_ord[r] = tid;
+  }
+  if constexpr (PART == 2) {
+    __syncthreads();
+    if (tid < n) wo[tid] = SD(s_ord[tid]);
+    for (int e = tid; e < n * n; e += GEP_NT) Xo[e] = GM(e % n, s_ord[e / n]);
+    return;
   }
   // X = U^-1 Z: rows from the last; column i of U staged (U(r, i), r <= i)
   if (tid < n) s_u[(n - 1) & 1][tid] = GU(tid, n - 1);
@@ -2623,7 +2735,7 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
     for (int i = 1; i < n; i++)
       if (fabs(GM(i, src)) > fabs(GM(pm, src))) pm = i;
     s_p[tid] = GM(pm, src) < 0.0 ? -1.0 : 1.0;
-    wo[tid] = s_d[src];
+    wo[tid] = SD(src);
   }
   __syncthreads();
   for (int e = tid; e < n * n; e += GEP_NT) {
@@ -2632,6 +2744,233 @@ __global__ __launch_bounds__(GEP_NT) void k_gep(const double* Ain,
   }
 #undef GM
 #undef GU
+#undef SE
+#undef SD
+}
+
+__device__ __forceinline__ double lane_bcast(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// Cholesky S = U^T U of an order in 132..256, in the registers of one
+// workgroup: thread (tr, tc) of 32 x 32 holds the entries (tr + 32 a, tc + 32
+// b), a <= b, of the symmetric matrix.  Row j of the trailing block goes
+// through LDS (one barrier a step; the owners of row j + 1 publish it as soon
+// as it is updated).  U to the upper triangle of the array, U^T below.  In
+// memory every step read and wrote the whole trailing block at the L1's rate,
+// 1.25 ms at n = 200; here
+// 0.18 ms.
+__global__ __launch_bounds__(1024) void k_gep_chol(const double* S, int n,
+                                                   double* U, int* err) {
+  __shared__ double row[2][MLCP_BMAX];
+  const int tid = threadIdx.x, tr = tid & 31, tc = tid >> 5;
+  double m[8][8];
+#pragma unroll
+  for (int a = 0; a < 8; a++)
+#pragma unroll
+    for (int b = a; b < 8; b++) {
+      const int i = min(tr + 32 * a, n - 1), c = min(tc + 32 * b, n - 1);
+      m[a][b] = S[min(i, c) + (long)max(i, c) * n];
+    }
+  if (tr == 0) {
+#pragma unroll
+    for (int b = 0; b < 8; b++) row[0][tc + 32 * b] = m[0][b];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int ja = 0; ja < 8; ja++) {
+    const int jend = min(32, n - 32 * ja);
+    for (int jr = 0; jr < jend; jr++) {
+      const int j = 32 * ja + jr;
+      const double* rj = row[j & 1];
+      double* rn = row[(j + 1) & 1];
+      const double d = rj[j];   // the same value in every thread
+      if (!(d > 0.0)) {
+        if (tid == 0) atomicOr(err, 4);
+        return;
+      }
+      const double di = 1.0 / d;
+      if (tid >= j && tid < n) {
+        const double u = sqrt(d);
+        U[tid + (long)j * n] = tid == j ? u : rj[tid] / u;
+      }
+      // rows and columns up to j of the block change too; nothing reads them
+      double ai[8], wc[8];
+#pragma unroll
+      for (int a = ja; a < 8; a++) {
+        ai[a] = rj[tr + 32 * a];
+        wc[a] = rj[tc + 32 * a] * di;
+      }
+#pragma unroll
+      for (int a = ja; a < 8; a++)
+#pragma unroll
+        for (int b = a; b < 8; b++) m[a][b] = fma(-ai[a], wc[b], m[a][b]);
+      if (jr < 31) {
+        if (tr == jr + 1) {
+#pragma unroll
+          for (int b = ja; b < 8; b++) rn[tc + 32 * b] = m[ja][b];
+        }
+      } else if (ja < 7) {
+        if (tr == 0) {
+#pragma unroll
+          for (int b = ja + 1; b < 8; b++) rn[tc + 32 * b] = m[ja + 1 < 8 ? ja + 1 : 7][b];
+        }
+      }
+      __syncthreads();
+    }
+  }
+  for (int e = tid; e < n * n; e += 1024) {
+    const int i = e % n, j = e / n;
+    if (i < j) U[e] = U[j + (long)i * n];
+  }
+}
+
+// Rows and columns of C = U^-T A U^-1 where the matrix exceeds LDS (k_gep's
+// U with U^T below its diagonal): x U = a by forward substitution, one wave
+// per row R, four entries c = lane + 64 q a lane, the rows of U prefetched
+// four steps ahead.  PASS 0 takes the rows of the symmetric A and leaves the
+// rows of A U^-1 in M, PASS 1 takes M's columns and replaces them.  The rows
+// are independent, so the device's other CUs share them: 26 us a pass at n =
+// 200 (3.1 ms for both by one workgroup sweeping the matrix row by row).
+template <int PASS>
+__global__ __launch_bounds__(256) void k_gep_subst(const double* A, int n,
+                                                   const double* U, double* M,
+                                                   const int* err) {
+  const int R = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (R >= n || (*err & 12)) return;
+  double a[4], x[4];
+  int c[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    c[q] = min(lane + 64 * q, n - 1);
+    a[q] = PASS == 0 ? A[min(R, c[q]) + (long)max(R, c[q]) * n]
+                     : M[c[q] + (long)R * n];
+    x[q] = 0.0;
+  }
+  double u[4][4], ud[4];
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    const long col = (long)min(b, n - 1) * n;
+#pragma unroll
+    for (int q = 0; q < 4; q++) u[b][q] = U[c[q] + col];
+    ud[b] = U[min(b, n - 1) + col];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int jend = min(64, n - 64 * q);
+    for (int j0 = 0; j0 < jend; j0 += 4) {
+      double un[4][4], udn[4];
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const int j = min(64 * q + j0 + 4 + b, n - 1);
+#pragma unroll
+        for (int r = q; r < 4; r++) un[b][r] = U[c[r] + (long)j * n];
+        udn[b] = U[j + (long)j * n];
+      }
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        // entries at or before j take part too, but are final (in x)
+        const double t = lane_bcast(a[q], j0 + b) / ud[b];
+        if (j0 + b < jend) {   // uniform
+          x[q] = lane == j0 + b ? t : x[q];
+#pragma unroll
+          for (int r = q; r < 4; r++) a[r] = fma(-t, u[b][r], a[r]);
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+#pragma unroll
+        for (int r = q; r < 4; r++) u[b][r] = un[b][r];
+        ud[b] = udn[b];
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (lane + 64 * q < n)
+      M[PASS == 0 ? R + (long)c[q] * n : c[q] + (long)R * n] = x[q];
+}
+
+// Eigenvectors from those of the tridiagonal matrix (columns of X, in place),
+// one wave per column: z = H_0 ... H_{n-3} z with the vectors sqrt(b) v below
+// U's diagonal, x = U^-1 z by back substitution, sign (largest |x|, the first
+// of ties, positive).  0.1 ms at n = 200; forming Q and sweeping the columns
+// together in one workgroup took 3.4 ms.
+__global__ __launch_bounds__(256) void k_gep_back(int n, const double* U,
+                                                  double* X, const int* err) {
+  const int cx = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (cx >= n || (*err & 12)) return;
+  double z[4], x[4];
+  int c[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    c[q] = min(lane + 64 * q, n - 1);
+    z[q] = ld_or0(X + c[q] + (long)cx * n, lane + 64 * q < n);
+    x[q] = 0.0;
+  }
+  for (int k0 = n - 3; k0 >= 0; k0 -= 4) {
+    double v[4][4];
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      const int k = k0 - b;
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        v[b][q] = ld_or0(U + c[q] + (long)max(k, 0) * n,
+                         k >= 0 && lane + 64 * q > k && lane + 64 * q < n);
+    }
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      double s = 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; q++) s = fma(v[b][q], z[q], s);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+#pragma unroll
+      for (int q = 0; q < 4; q++) z[q] = fma(-s, v[b][q], z[q]);
+    }
+  }
+#pragma unroll
+  for (int q = 3; q >= 0; q--) {
+    const int jend = min(64, n - 64 * q);   // none: <= 0
+    for (int j0 = jend - 1; j0 >= 0; j0 -= 4) {
+      double u[4][4], ud[4];
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const int j = 64 * q + max(j0 - b, 0);
+#pragma unroll
+        for (int r = 0; r <= q; r++) u[b][r] = U[c[r] + (long)j * n];
+        ud[b] = U[j + (long)j * n];
+      }
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        if (j0 - b >= 0) {   // uniform
+          const double t = lane_bcast(z[q], j0 - b) / ud[b];
+          x[q] = lane == j0 - b ? t : x[q];
+#pragma unroll
+          for (int r = 0; r <= q; r++) z[r] = fma(-t, u[b][r], z[r]);
+        }
+      }
+    }
+  }
+  double m = 0.0;
+#pragma unroll
+  for (int q = 0; q < 4; q++) m = fmax(m, fabs(x[q]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+  double sg = 1.0;
+  bool found = false;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const unsigned long long at = __ballot(fabs(x[q]) == m && lane + 64 * q < n);
+    if (at && !found) {
+      sg = lane_bcast(x[q], __ffsll((long long)at) - 1) < 0.0 ? -1.0 : 1.0;
+      found = true;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (lane + 64 * q < n) X[c[q] + (long)cx * n] = sg * x[q];
 }
 
 // --------------------------------------------------------------------------

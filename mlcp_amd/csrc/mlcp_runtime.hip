@@ -156,7 +156,7 @@ static int setup_kernels() {
                       NX_KERNELS2(k_op_solve, 3),  NX_KERNELS2(k_op_solve, 4),
                       (const void*)k_lc_solve<1>,  (const void*)k_lc_solve<2>,
                       (const void*)k_lc_solve<3>,  (const void*)k_lc_solve<4>,
-                      (const void*)k_gep<1>};
+                      (const void*)k_gep<1, 0>};
 #undef NX_KERNELS2
 #undef NX_KERNELS
   g_lds_dev = (size_t)v;
@@ -1272,25 +1272,45 @@ static int phase_ortho(mlcp_session* s, int nals) {
   return 0;
 }
 
-// LDS placement of the eigensolver's work matrices (k_gep MODE) for order n
-// and the dynamic LDS it needs.
-static int gep_mode(int n, size_t* lds) {
-  // the working matrix in LDS with the odd leading dimension n | 1
+// Dynamic LDS of the eigensolver's working matrix (odd leading dimension n |
+// 1) for order n; 0 where it does not fit and stays in ws.
+static size_t gep_lds(int n) {
   const size_t mc = (size_t)n * (n | 1) * sizeof(double);
-  if (mc <= lds_limit((const void*)k_gep<1>)) { *lds = mc; return 1; }
-  *lds = 0;
-  return 0;
+  return mc <= lds_limit((const void*)k_gep<1, 0>) ? mc : 0;
 }
 
-#define LAUNCH_GEP(kid, n, ...)                                             \
-  do {                                                                    \
-    size_t lds_;                                                          \
-    const int mode_ = gep_mode(n, &lds_);                                 \
-    if (mode_ == 1)                                                       \
-      PLAUNCH(kid, k_gep<1>, dim3(1), dim3(1024), lds_, __VA_ARGS__);     \
-    else                                                                  \
-      PLAUNCH(kid, k_gep<0>, dim3(1), dim3(1024), lds_, __VA_ARGS__);     \
+// The eigensolver on stream st (k_gep's arguments), timed by the events e0
+// and e1 if given.
+static void launch_gep(hipStream_t st, const double* A, const double* S, int n,
+                       double* ws, double* X, double* w, int* err,
+                       hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
+#define GEP_LAUNCH(kern, grid, block, lds, ea, eb, ...)                      \
+  do {                                                                      \
+    if (ea || eb)                                                           \
+      hipExtLaunchKernelGGL(kern, grid, block, lds, st, ea, eb, 0,          \
+                            __VA_ARGS__);                                   \
+    else                                                                    \
+      hipLaunchKernelGGL(kern, grid, block, lds, st, __VA_ARGS__);          \
   } while (0)
+  const hipEvent_t none = nullptr;
+  const size_t lds = gep_lds(n);
+  if (lds) {
+    GEP_LAUNCH((k_gep<1, 0>), dim3(1), dim3(GEP_NT), lds, e0, e1, A, S, n, ws,
+               X, w, err);
+    return;
+  }
+  const dim3 rows((n + 3) / 4);
+  double* M = ws + (size_t)n * n;
+  const double* U = ws;
+  const int* er = err;
+  GEP_LAUNCH(k_gep_chol, dim3(1), dim3(1024), 0, e0, none, S, n, ws, err);
+  GEP_LAUNCH(k_gep_subst<0>, rows, dim3(256), 0, none, none, A, n, U, M, er);
+  GEP_LAUNCH(k_gep_subst<1>, rows, dim3(256), 0, none, none, A, n, U, M, er);
+  GEP_LAUNCH((k_gep<0, 2>), dim3(1), dim3(GEP_NT), 0, none, none, A, S, n, ws,
+             X, w, err);
+  GEP_LAUNCH(k_gep_back, rows, dim3(256), 0, none, e1, n, U, X, er);
+#undef GEP_LAUNCH
+}
 
 static int phase_gep(mlcp_session* s) {
   int B = s->nbloc;
@@ -1299,9 +1319,10 @@ static int phase_gep(mlcp_session* s) {
   PLAUNCH(KID_PAIR_INNER, k_pair_inner, dim3(s->npj), dim3(MLCP_NT), 0,
           s->pool, (const PairJob*)s->pj.p, s->QHQ.p);
   // QHQ at QHQ.p + B*B, S at QHQ.p
-  LAUNCH_GEP(KID_GEP, B,
-          (const double*)(s->QHQ.p + (size_t)B * B), (const double*)s->QHQ.p,
-          B, s->ws.p, s->U.p, s->eig.p, s->err.p);
+  hipEvent_t e0, e1;
+  probe_events(s, KID_GEP, &e0, &e1);
+  launch_gep(s->st, s->QHQ.p + (size_t)B * B, s->QHQ.p, B, s->ws.p, s->U.p,
+             s->eig.p, s->err.p, e0, e1);
   HCHK(hipGetLastError());
   return 0;
 }
@@ -2490,14 +2511,7 @@ extern "C" int mlcp_hip_gep(int n, const double* A, const double* Bm,
   HCHK(hipMemcpy(dB, Bm, nn * sizeof(double), hipMemcpyHostToDevice));
   HCHK(hipMemset(e.p, 0, sizeof(int)));
   if (setup_kernels()) return -1;
-  size_t lds = 0;
-  const int mode = gep_mode(n, &lds);
-  if (mode == 1)
-    hipLaunchKernelGGL(k_gep<1>, dim3(1), dim3(1024), lds, 0, dA, dB, n, ws,
-                       dX, dw, e.p);
-  else
-    hipLaunchKernelGGL(k_gep<0>, dim3(1), dim3(1024), lds, 0, dA, dB, n, ws,
-                       dX, dw, e.p);
+  launch_gep(0, dA, dB, n, ws, dX, dw, e.p);
   HCHK(hipGetLastError());
   int err = 0;
   HCHK(hipMemcpy(&err, e.p, sizeof(int), hipMemcpyDeviceToHost));
@@ -2551,14 +2565,7 @@ extern "C" int mlcp_hip_gep_noalloc(int n, const double* dA, const double* dB,
   // info is an output: cleared by a fill kernel (capturable), then error
   // bits are or-ed in by the eigensolver
   hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, dinfo, 1L, 0);
-  size_t lds = 0;
-  const int mode = gep_mode(n, &lds);
-  if (mode == 1)
-    hipLaunchKernelGGL(k_gep<1>, dim3(1), dim3(1024), lds, st, dA, dB, n, ws,
-                       dX, dw, dinfo);
-  else
-    hipLaunchKernelGGL(k_gep<0>, dim3(1), dim3(1024), lds, st, dA, dB, n, ws,
-                       dX, dw, dinfo);
+  launch_gep(st, dA, dB, n, ws, dX, dw, dinfo);
   HCHK(hipGetLastError());
   return 0;
 }
