@@ -117,6 +117,10 @@ struct LcArgs {
   int nchunk;            // old-column chunks of LC_CHUNK
   int ngrp;              // groups of LC_GRP chunks: partial sums per target
   double* X;             // [B][ndof][xr * ncold]  X(i,c) = <F_i^d, O_c^d>
+  // modes [gb, ge) whose X the right-hand side reads one by one; the product
+  // of the other modes' X is in O ([B][xr * ncold]; nullptr: all modes)
+  int gb, ge;
+  double* O;
   double* G;             // [B][ndof][rstr]
   double* part;          // [B][ngrp][Rmax * nmax] partial right-hand sides
   int pstr;              // Rmax * nmax

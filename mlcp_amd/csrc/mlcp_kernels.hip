@@ -1734,85 +1734,77 @@ __global__ void k_lc_weights(double* w, const double* U, int ldU,
   }
 }
 
-// X[t][d](i,c) = <F_i^d, O_c^d> for a chunk of 64 old columns; chunk 0 also
-// refreshes G[t][d].  job = (t, chunk).  The cross Grams are an R x 64 x n
-// matrix product on the FP64 matrix cores: wave g owns the 16 old columns
-// [16g, 16g+16) of the chunk for every row tile of the target, the basis
-// runs in k-steps of 4 (operands loaded eight k-steps ahead), and the result
-// tiles pass through the wave's LDS so that each column of X is written as
-// runs of consecutive rows.
+// X[t][d](i,c) = <F_i^d, O_c^d> for cpw chunks of 64 old columns of target t;
+// the workgroup of the first chunk also refreshes G[t][d].  The cross Grams are
+// an R x 64 cpw x n matrix product on the FP64 matrix cores.  The target's
+// factors go through LDS once for the whole workgroup (rows of S doubles, S an
+// odd multiple of 4, so that sixteen rows and four k fall into different
+// banks); a wave owns sixteen old columns at a time, for every row tile, and
+// reads them from memory four k at once.  The columns are the rows of the
+// result tile: its four registers are runs of sixteen consecutive entries of
+// X, stored as they are.  200 targets of rank 16-64, 7965 columns of 120: 0.63
+// ms (0.91 with the factors read by every wave and the tiles transposed
+// through LDS); the matrix cores would take 0.26, the stores 0.1.
 template <int RTM>
-__global__ __launch_bounds__(MLCP_NT, RTM < 4 ? 4 : 2) void k_lc_refresh(LcArgs a,
-                                                         const int2* jobs,
-                                                         int d) {
-  __shared__ double Ts[4][16 * 65];   // per wave: 16 columns x 64 rows (+1)
-  int2 jb = jobs[blockIdx.x];
-  if (a.done && a.done[jb.x]) return;   // converged target (tolerance form)
-  int t = jb.x, ch = jb.y, R = a.R[t], n = a.p.nbas[d];
-  int c0 = ch * LC_CHUNK, nc = min(LC_CHUNK, a.ncold - c0);
+__global__ __launch_bounds__(2 * MLCP_NT) void k_lc_refresh(LcArgs a, int cpw,
+                                                            int d) {
+  extern __shared__ double Fs[];
+  const int nwg = (a.nchunk + cpw - 1) / cpw;
+  const int t = blockIdx.x / nwg, ch = (blockIdx.x - t * nwg) * cpw;
+  if (a.done && a.done[t]) return;   // converged target (tolerance form)
+  const int R = a.R[t], n = a.p.nbas[d], S = (((n + 3) >> 2) | 1) << 2;
   double* X = a.X + ((long)t * a.p.ndof + d) * ((long)a.xr * a.ncold);
   const int lane = TID & 63, lr = lane & 15, lq = lane >> 4;
   const int g = __builtin_amdgcn_readfirstlane(TID >> 6);
+  const int nw = blockDim.x >> 6;
   const int RT = (R + 15) >> 4;
-  if (16 * g < nc) {
-    // wave g: old columns 16g .. 16g+15 of the chunk, every row tile
-    const int cl = 16 * g + lr;
-    const bool cok = cl < nc;
-    const double* o = colp(a.p, d, a.ocol0 + c0 + (cok ? cl : 0));
-    const double* f[RTM];
-    bool iok[RTM];
+  for (int i = g; i < R; i += nw) {
+    const double* f = colp(a.p, d, a.col[t] + i);
+    for (int m = lane; m < n; m += 64) Fs[i * S + m] = f[m];
+  }
+  __syncthreads();
+  const double* fr[RTM];
 #pragma unroll
-    for (int rt = 0; rt < RTM; rt++) {
-      const int ia = 16 * rt + lr;
-      iok[rt] = rt < RT && ia < R;
-      f[rt] = colp(a.p, d, a.col[t] + (iok[rt] ? ia : 0));
-    }
+  for (int rt = 0; rt < RTM; rt++) fr[rt] = Fs + min(16 * rt + lr, R - 1) * S;
+  const int cend = min(a.ncold, (ch + cpw) * LC_CHUNK);
+  for (int c0 = ch * LC_CHUNK + 16 * g; c0 < cend; c0 += 16 * nw) {
+    // (columns past cend and rows past R give results that are not stored)
+    const double* o = colp(a.p, d, a.ocol0 + min(c0 + lr, cend - 1));
     v4d acc[RTM];
 #pragma unroll
     for (int rt = 0; rt < RTM; rt++) acc[rt] = (v4d){0.0, 0.0, 0.0, 0.0};
     const int nks = (n + 3) >> 2;
     for (int ks0 = 0; ks0 < nks; ks0 += 8) {
-      double bv[8], av[8][RTM];
+      double ov[8];
 #pragma unroll
       for (int b = 0; b < 8; b++) {
-        const int m = 4 * (ks0 + b) + lq, mc = min(m, n - 1);
-        bv[b] = ld_or0(o + mc, cok && m < n);
-#pragma unroll
-        for (int rt = 0; rt < RTM; rt++) av[b][rt] = ld_or0(f[rt] + mc, iok[rt] && m < n);
+        const int m = 4 * (ks0 + b) + lq;
+        ov[b] = ld_or0(o + min(m, n - 1), m < n);
       }
-      // (zero operands past R and n: no guard between the MFMAs)
 #pragma unroll
-      for (int b = 0; b < 8; b++)
+      for (int b = 0; b < 8; b++) {
+        const int mc = min(4 * (ks0 + b) + lq, n - 1);   // zero operand past n
 #pragma unroll
-        for (int rt = 0; rt < RTM; rt++) acc[rt] = mfma_f64_4(av[b][rt], bv[b], acc[rt]);
+        for (int rt = 0; rt < RTM; rt++) acc[rt] = mfma_f64_4(ov[b], fr[rt][mc], acc[rt]);
+      }
     }
-    // element v of lane l: row 16rt + l/16 + 4v, column 16g + l%16; the
-    // tile goes through this wave's LDS so that the stores run along rows
-    double* ts = Ts[g];
+    // element v: column c0 + l/16 + 4v, row 16rt + l%16
 #pragma unroll
-    for (int rt = 0; rt < RTM; rt++)
-      if (rt < RT) {
+    for (int rt = 0; rt < RTM; rt++) {
+      const int i = 16 * rt + lr;
 #pragma unroll
-        for (int v = 0; v < 4; v++) ts[lr * 65 + 16 * rt + lq + 4 * v] = acc[rt][v];
+      for (int v = 0; v < 4; v++) {
+        const int c = c0 + lq + 4 * v;
+        if (i < R && c < cend) X[(long)c * a.xr + i] = acc[rt][v];
       }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // the wave's 16 columns are one contiguous block of 16 xr doubles of X:
-    // store j writes its doubles 64j .. 64j + 63, one per lane
-    double* xb = X + (long)(c0 + 16 * g) * a.xr;
-    const int xr = a.xr, tot = min(16, nc - 16 * g) * xr;
-    for (int f = lane; f < tot; f += 64) {
-      const int col = f / xr, row = f - col * xr;
-      if (row < R) xb[f] = ts[col * 65 + row];
     }
   }
   if (ch == 0) {
     // own Gram G(l, i) = <F_l^d, F_i^d>: tile (lt, it) of the RT x RT grid
-    // on wave (lt*RT + it) % 4
+    // on wave (lt*RT + it) % nw
     double* G = a.G + ((long)t * a.p.ndof + d) * a.rstr;
     const int nks = (n + 3) >> 2;
-    for (int q = g; q < RT * RT; q += 4) {
+    for (int q = g; q < RT * RT; q += nw) {
       const int lt = q / RT, it = q % RT;
       const int la = 16 * lt + lr, ib = 16 * it + lr;
       const double* fl = colp(a.p, d, a.col[t] + (la < R ? la : 0));
@@ -1839,6 +1831,39 @@ __global__ __launch_bounds__(MLCP_NT, RTM < 4 ? 4 : 2) void k_lc_refresh(LcArgs 
   }
 }
 
+// O(i,c) = prod_{d < gb or d >= ge} X_d(i,c) of target t over a chunk of old
+// columns: the modes that stay as they are while the steps
+// of modes [gb, ge) run.  The right-hand side is bound by its reads of X (11
+// modes of 0.5 GB each at 200 targets of rank 16-64, 12 modes: 1.87 ms a
+// step); with four modes to a group it reads O and three modes (1.03 ms), and
+// this product is formed once in four steps (1.17 ms).  120 targets of rank
+// 32, 8 modes in threes: 200 us -> 125 and 150 every third step.
+__global__ __launch_bounds__(MLCP_NT) void k_lc_outer(LcArgs a) {
+  const int t = blockIdx.x / a.nchunk, ch = blockIdx.x - t * a.nchunk;
+  if (a.done && a.done[t]) return;   // converged target (tolerance form)
+  const int R = a.R[t], D = a.p.ndof, c0 = ch * LC_CHUNK;
+  const int nc = min(LC_CHUNK, a.ncold - c0), ng = a.ge - a.gb, no = D - ng;
+  const long xs = (long)a.xr * a.ncold;
+  const double* X = a.X + (long)t * D * xs + (long)c0 * a.xr;
+  double* O = a.O + (long)t * xs + (long)c0 * a.xr;
+  for (int e = TID; e < nc * R; e += MLCP_NT) {
+    const int off = (e / R) * a.xr + e % R;
+    double p = 1.0;
+    for (int m0 = 0; m0 < no; m0 += 4) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int m = min(m0 + u, no - 1);
+        v[u] = X[(m < a.gb ? m : m + ng) * xs + off];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        if (m0 + u < no) p *= v[u];
+    }
+    O[off] = p;
+  }
+}
+
 // partial right-hand side of target t over one group of LC_GRP chunks of
 // old columns: part(i,m) = sum_c w_c cO_c prod_{d!=k} X_d(i,c) O_c^k(m),
 // summed over the group's chunks in the MFMA accumulators, so that each
@@ -1857,8 +1882,12 @@ __global__ __launch_bounds__(MLCP_NT) void k_lc_rhs(LcArgs a, int k) {
   const int lane = TID & 63, lr = lane & 15, lq = lane >> 4;
   const int g = __builtin_amdgcn_readfirstlane(TID >> 6);
   const int RT = (R + 15) >> 4, CT = (n + 15) >> 4;
-  // output tile q = g + 4 tq of the RT x CT grid (CT <= 8) in acct[tq]
+  // Output tile acct[tq] of the RT x CT grid (CT <= 8).  From four column
+  // tiles on a wave owns the column tiles g and g + 4 for every row tile (tq =
+  // RTM j + rt), so that an old column is read once for all of them; below
+  // that the tiles are dealt out, q = g + 4 tq.  The sums are the same.
   constexpr int TPW = 2 * RTM;
+  const bool bycol = CT >= 4;
   v4d acct[TPW];
 #pragma unroll
   for (int tq = 0; tq < TPW; tq++) acct[tq] = (v4d){0.0, 0.0, 0.0, 0.0};
@@ -1881,17 +1910,26 @@ __global__ __launch_bounds__(MLCP_NT) void k_lc_rhs(LcArgs a, int k) {
       off[j] = (c0 + c) * a.xr + i;
       pr[j] = ok ? w[c0 + c] * a.p.coef[a.ocol0 + c0 + c] : 0.0;
     }
-    for (int m0 = 1; m0 < D; m0 += MG) {
+    if (a.O) {   // the modes outside the group
+      const double* Om = a.O + (long)t * xs;
+      double v[PE];
+#pragma unroll
+      for (int j = 0; j < PE; j++) v[j] = Om[off[j]];
+#pragma unroll
+      for (int j = 0; j < PE; j++) pr[j] *= v[j];
+    }
+    const int ng = a.ge - a.gb, kg = k - a.gb;
+    for (int m0 = 1; m0 < ng; m0 += MG) {
       double v[MG][PE];
 #pragma unroll
       for (int gm = 0; gm < MG; gm++) {
-        const double* Xm = X + (long)((k + min(m0 + gm, D - 1)) % D) * xs;
+        const double* Xm = X + (long)(a.gb + (kg + min(m0 + gm, ng - 1)) % ng) * xs;
 #pragma unroll
         for (int j = 0; j < PE; j++) v[gm][j] = Xm[off[j]];
       }
 #pragma unroll
       for (int gm = 0; gm < MG; gm++)
-        if (m0 + gm < D) {
+        if (m0 + gm < ng) {
 #pragma unroll
           for (int j = 0; j < PE; j++) pr[j] *= v[gm][j];
         }
@@ -1906,6 +1944,34 @@ __global__ __launch_bounds__(MLCP_NT) void k_lc_rhs(LcArgs a, int k) {
     // += sum_c P(c, i) O_c^k(m) on the FP64 matrix cores; a k-step is four
     // old columns (P rows past nc are never read: the operand is zero)
     const int nks = (nc + 3) >> 2;
+    if (bycol) {
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int ct = g + 4 * j, mcol = 16 * ct + lr;
+        if (ct >= CT) continue;   // uniform
+        const bool mok = mcol < n;
+        const int mc = min(mcol, n - 1);
+        for (int ks0 = 0; ks0 < nks; ks0 += 4) {
+          double av[4][RTM], bv[4];
+#pragma unroll
+          for (int b = 0; b < 4; b++) {
+            const int c = 4 * (ks0 + b) + lq, cc = min(c, nc - 1);
+            bv[b] = ld_or0(colp(a.p, k, a.ocol0 + c0 + cc) + mc, c < nc && mok);
+#pragma unroll
+            for (int rt = 0; rt < RTM; rt++) {
+              const int i = 16 * rt + lr;
+              av[b][rt] = ld_or0(P + cc * R + min(i, R - 1), c < nc && i < R);
+            }
+          }
+#pragma unroll
+          for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int rt = 0; rt < RTM; rt++)
+              acct[RTM * j + rt] = mfma_f64_4(av[b][rt], bv[b], acct[RTM * j + rt]);
+        }
+      }
+      continue;
+    }
 #pragma unroll
     for (int tq = 0; tq < TPW; tq++) {
       const int q = g + 4 * tq;
@@ -1935,8 +2001,9 @@ __global__ __launch_bounds__(MLCP_NT) void k_lc_rhs(LcArgs a, int k) {
 #pragma unroll
   for (int tq = 0; tq < TPW; tq++) {
     const int q = g + 4 * tq;
-    if (q < RT * CT) {
-      const int rt = q % RT, ct = q / RT, mcol = 16 * ct + lr;
+    const int rt = bycol ? tq % RTM : q % RT;
+    const int ct = bycol ? g + 4 * (tq / RTM) : q / RT, mcol = 16 * ct + lr;
+    if (ct < CT && rt < RT) {
       // element v of lane l: row 16rt + l/16 + 4v, column 16ct + l%16
 #pragma unroll
       for (int v = 0; v < 4; v++) {

@@ -154,6 +154,8 @@ static int setup_kernels() {
                       NX_KERNELS2(k_gs_state, 3), NX_KERNELS2(k_gs_state, 4),
                       NX_KERNELS2(k_op_solve, 1),  NX_KERNELS2(k_op_solve, 2),
                       NX_KERNELS2(k_op_solve, 3),  NX_KERNELS2(k_op_solve, 4),
+                      (const void*)k_lc_refresh<2>, (const void*)k_lc_refresh<3>,
+                      (const void*)k_lc_refresh<4>,
                       (const void*)k_lc_solve<1>,  (const void*)k_lc_solve<2>,
                       (const void*)k_lc_solve<3>,  (const void*)k_lc_solve<4>,
                       (const void*)k_gep<1, 0>};
@@ -255,9 +257,7 @@ struct mlcp_session {
   int gs_xst = 1;
   DBuf<int> d_hsp;
   // linear-combination ALS
-  DBuf<double> lcX, lcG, lcPart, lcW;
-  DBuf<int2> lcJobs;
-  int lc_jobs_b = -1, lc_jobs_c = -1;   // shape of the uploaded job list
+  DBuf<double> lcX, lcO, lcG, lcPart, lcW;
   // GEP
   DBuf<double> QHQ, S, U, eig, ws;
   DBuf<PairJob> pj;
@@ -1327,6 +1327,16 @@ static int phase_gep(mlcp_session* s) {
   return 0;
 }
 
+// Modes to a group of the update's right-hand sides (k_lc_outer), or D for
+// none, for B targets of rank up to R and N old columns: where X exceeds the
+// 256 MB last-level cache and there are modes enough to save reads.  A step
+// reads g arrays and its share of the product's D - g + 1, instead of D - 1: 5
+// of 7 for eight modes in threes, 6.25 of 11 for twelve in fours.
+static int lc_group(double D, double B, double R, double N) {
+  if (D < 6 || 8 * D * B * R * N < 512e6) return (int)D;
+  return D < 12 ? 3 : 4;
+}
+
 static LcArgs lc_args(mlcp_session* s, int B, const int* col, const int* R,
                       int xr, int ocol0, int ncold) {
   LcArgs a;
@@ -1343,6 +1353,9 @@ static LcArgs lc_args(mlcp_session* s, int B, const int* col, const int* R,
   a.nchunk = (ncold + LC_CHUNK - 1) / LC_CHUNK;
   a.ngrp = (a.nchunk + LC_GRP - 1) / LC_GRP;
   a.X = s->lcX.p;
+  a.gb = 0;
+  a.ge = s->ndof;
+  a.O = nullptr;
   a.G = s->lcG.p;
   a.part = s->lcPart.p;
   a.pstr = s->Rmax * s->nmax;
@@ -1353,38 +1366,42 @@ static LcArgs lc_args(mlcp_session* s, int B, const int* col, const int* R,
   return a;
 }
 
-// k_lc_refresh for the row tiles of the block's largest rank
-#define LC_REFRESH_LAUNCH(grid, block, lds, ...)                            \
-  do {                                                                    \
-    if (s->Rmax <= 32)                                                    \
-      PLAUNCH(KID_LC_REFRESH, k_lc_refresh<2>, grid, block, lds, __VA_ARGS__); \
-    else if (s->Rmax <= 48)                                               \
-      PLAUNCH(KID_LC_REFRESH, k_lc_refresh<3>, grid, block, lds, __VA_ARGS__); \
-    else                                                                  \
-      PLAUNCH(KID_LC_REFRESH, k_lc_refresh<4>, grid, block, lds, __VA_ARGS__); \
-  } while (0)
+// k_lc_refresh of mode d for the row tiles of the block's largest rank.  A
+// workgroup takes up to four chunks of old columns, as many as leave two
+// workgroups a CU (one chunk by four waves, more by eight): the staging of the
+// target's factors is paid once for them.
+static void launch_lc_refresh(mlcp_session* s, const LcArgs& a, int d) {
+  const int cpw = std::max(1, std::min(4, a.B * a.nchunk / (2 * g_cus)));
+  const dim3 grid(a.B * ((a.nchunk + cpw - 1) / cpw));
+  const dim3 block(cpw > 1 ? 2 * MLCP_NT : MLCP_NT);
+  const int S = (((s->nbas[d] + 3) / 4) | 1) * 4;
+  const size_t lds = (size_t)s->Rmax * S * sizeof(double);
+  switch ((s->Rmax + 15) / 16) {
+    case 1:
+    case 2:
+      PLAUNCH(KID_LC_REFRESH, k_lc_refresh<2>, grid, block, lds, a, cpw, d);
+      break;
+    case 3:
+      PLAUNCH(KID_LC_REFRESH, k_lc_refresh<3>, grid, block, lds, a, cpw, d);
+      break;
+    default:
+      PLAUNCH(KID_LC_REFRESH, k_lc_refresh<4>, grid, block, lds, a, cpw, d);
+  }
+}
 
-// Linear-combination ALS sweeps on the prepared LcArgs (weights in lcW,
-// penalties in d_pen).
 static int lc_als(mlcp_session* s, LcArgs& a, int nitn, bool final_norm) {
   int D = s->ndof, B = a.B;
-  // job list (target, chunk of old columns), uploaded when it changes (so a
-  // captured cycle holds no host copy)
-  const int nj = B * a.nchunk;
-  if (s->lc_jobs_b != B || s->lc_jobs_c != a.nchunk) {
-    std::vector<int2> jobs;
-    for (int t = 0; t < B; t++)
-      for (int c = 0; c < a.nchunk; c++) jobs.push_back(make_int2(t, c));
-    if (s->lcJobs.put(jobs, s->st)) return -1;
-    s->lc_jobs_b = B;
-    s->lc_jobs_c = a.nchunk;
-  }
-  for (int d = 0; d < D; d++) {
-    LC_REFRESH_LAUNCH( dim3(nj), dim3(MLCP_NT), 0, a,
-            (const int2*)s->lcJobs.p, d);
-  }
+  for (int d = 0; d < D; d++) launch_lc_refresh(s, a, d);
+  const int grp = s->lcO.p ? lc_group(D, B, s->Rmax, a.ncold) : D;
   for (int it = 0; it < nitn; it++)
     for (int k = 0; k < D; k++) {
+      if (grp < D && k % grp == 0) {
+        a.gb = k;
+        a.ge = std::min(D, k + grp);
+        a.O = s->lcO.p;
+        hipLaunchKernelGGL(k_lc_outer, dim3(B * a.nchunk), dim3(MLCP_NT), 0,
+                           s->st, a);
+      }
       if (s->Rmax <= 16)
         PLAUNCH(KID_LC_RHS, k_lc_rhs<1>, dim3(B * a.ngrp), dim3(MLCP_NT), 0,
                 a, k);
@@ -1408,8 +1425,7 @@ static int lc_als(mlcp_session* s, LcArgs& a, int nitn, bool final_norm) {
       else
         PLAUNCH(KID_LC_SOLVE, k_lc_solve<4>, dim3(B), dim3(MLCP_NT), lds_s, a, k);
       if (!(it == nitn - 1 && k == D - 1)) {
-        LC_REFRESH_LAUNCH( dim3(nj), dim3(MLCP_NT), 0, a,
-                (const int2*)s->lcJobs.p, k);
+        launch_lc_refresh(s, a, k);
         if (a.done && k == D - 1)
           hipLaunchKernelGGL(k_lc_conv, dim3(B), dim3(MLCP_NT), 0, s->st, a,
                              it);
@@ -1433,7 +1449,9 @@ static int phase_update(mlcp_session* s, const double* Ud, int nals) {
       s->lcG.need((size_t)B * D * s->Rmax * s->Rmax) ||
       s->lcPart.need((size_t)B * ((N + LC_CHUNK - 1) / LC_CHUNK) * s->Rmax *
                      s->nmax) ||
-      s->lcW.need((size_t)B * N))
+      s->lcW.need((size_t)B * N) ||
+      (!s->oneshot && lc_group(D, B, s->Rmax, N) < D &&
+       s->lcO.need((size_t)B * s->Rmax * N)))
     return -1;
   hipLaunchKernelGGL(k_lc_weights, dim3(256), dim3(256), 0, s->st, s->lcW.p,
                      Ud, B, (const int*)s->d_colstate.p, N, B);
@@ -2754,7 +2772,7 @@ extern "C" void intwdevicemem_(const int* rk, const int* ndof,
   const double upd = *update
       ? 8 * (B * D * R * N + B * D * r2 +
              B * std::ceil(N / LC_CHUNK) * R * nmax + B * N) +
-            8 * B * std::ceil(N / LC_CHUNK)
+            (lc_group(D, B, R, N) < D ? 8 * B * R * N : 0.0)
       : 0.0;
   printf(" *** MI355X device memory requirements *** \n \n");
   printf(" Factor pool (4 regions)  : %10.2f MB \n", pool * MB);
