@@ -156,6 +156,8 @@ static int setup_kernels() {
                       NX_KERNELS2(k_op_solve, 3),  NX_KERNELS2(k_op_solve, 4),
                       (const void*)k_lc_refresh<2>, (const void*)k_lc_refresh<3>,
                       (const void*)k_lc_refresh<4>,
+                      (const void*)k_lc_fit<1>, (const void*)k_lc_fit<2>,
+                      (const void*)k_lc_fit<3>, (const void*)k_lc_fit<4>,
                       (const void*)k_lc_solve<1>,  (const void*)k_lc_solve<2>,
                       (const void*)k_lc_solve<3>,  (const void*)k_lc_solve<4>,
                       (const void*)k_gep<1, 0>};
@@ -1391,6 +1393,36 @@ static void launch_lc_refresh(mlcp_session* s, const LcArgs& a, int d) {
 
 static int lc_als(mlcp_session* s, LcArgs& a, int nitn, bool final_norm) {
   int D = s->ndof, B = a.B;
+  const int pk = s->probe_kid;
+  if (a.nchunk <= 2 && !a.done && pk != KID_LC_RHS && pk != KID_LC_SOLVE &&
+      pk != KID_LC_REFRESH) {
+    // (three chunks: 1.42 ms for a fit of 175 terms in 32 that takes 1.36 in
+    // steps); LDS: the largest of the steps' own
+    const int rt = (s->Rmax + 15) / 16;
+    const size_t R = s->Rmax, n1 = (s->nmax | 1), S = ((s->nmax + 3) / 4 | 1) * 4;
+    const size_t lds = std::max({R * S, R * n1 + R * R,
+                                 (size_t)LC_CHUNK * 16 * rt}) *
+                       sizeof(double);
+    switch (rt) {
+      case 1:
+        hipLaunchKernelGGL(k_lc_fit<1>, dim3(B), dim3(MLCP_NT), lds, s->st, a,
+                           nitn, final_norm ? 1 : 0);
+        break;
+      case 2:
+        hipLaunchKernelGGL(k_lc_fit<2>, dim3(B), dim3(MLCP_NT), lds, s->st, a,
+                           nitn, final_norm ? 1 : 0);
+        break;
+      case 3:
+        hipLaunchKernelGGL(k_lc_fit<3>, dim3(B), dim3(MLCP_NT), lds, s->st, a,
+                           nitn, final_norm ? 1 : 0);
+        break;
+      default:
+        hipLaunchKernelGGL(k_lc_fit<4>, dim3(B), dim3(MLCP_NT), lds, s->st, a,
+                           nitn, final_norm ? 1 : 0);
+    }
+    HCHK(hipGetLastError());
+    return 0;
+  }
   for (int d = 0; d < D; d++) launch_lc_refresh(s, a, d);
   const int grp = s->lcO.p ? lc_group(D, B, s->Rmax, a.ncold) : D;
   for (int it = 0; it < nitn; it++)

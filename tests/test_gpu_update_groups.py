@@ -71,3 +71,33 @@ def test_grouped_products(hip, D, n, B, R):
 def test_column_tiles(hip, D, n, B, R):
     print("[case] update tiles", D, n, B, R, flush=True)
     check(D, n, B, R, n + R)
+
+
+@pytest.mark.parametrize("n,R,old", [(1, 1, 1), (10, 8, 64), (17, 16, 65),
+                                     (33, 33, 128), (33, 33, 129),
+                                     (128, 64, 100)])
+def test_one_launch_fit(hip, n, R, old):
+    """Fits on both sides of two chunks of 64 old columns (one launch or one a
+    step): a vector of ``old`` columns that are R products, repeated with other
+    coefficients, has to come back as those products."""
+    from mlcp_amd.intertwine import gpu_als
+    print("[case] fit", n, R, old, flush=True)
+    D = 3
+    rng = np.random.default_rng(n + old)
+    fac = rng.normal(size=(R, D, n))
+    fac /= np.linalg.norm(fac, axis=2, keepdims=True)
+    which = np.arange(old) % R
+    gc = np.exp(rng.uniform(-1.0, 1.0, old))
+    want = np.zeros(R)
+    np.add.at(want, which, gc)
+    F0 = fac.reshape(R, D * n)
+    fc, fb = gpu_als(np.ones(R), F0.copy(), gc, F0[which].copy(),
+                     np.full(D, n, dtype=np.int32), 2)
+    got = np.asarray(fb).reshape(R, D, n)
+    S, M, G = np.ones((R, R)), np.ones((R, R)), np.ones((R, R))
+    for d in range(D):
+        S *= got[:, d] @ got[:, d].T
+        M *= got[:, d] @ fac[:, d].T
+        G *= fac[:, d] @ fac[:, d].T
+    cw = (fc @ M @ want) / np.sqrt((fc @ S @ fc) * (want @ G @ want))
+    assert abs(abs(cw) - 1.0) <= 1e-8
