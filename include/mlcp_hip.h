@@ -190,7 +190,8 @@ int mlcp_hip_session_set_warmstart(mlcp_session *s, mlcp_mlp *q);
  *   had_split  waves sharing each 64-element group of a Hadamard tile,
  *              each over its own range of the mode's sub-slots (1, 2, 4, 8
  *              or 16; had_tile/64 * had_split <= 16)
- *   gs_stride  Gram-Schmidt workgroup stride (1: all CUs, 8: one XCD)
+ *   gs_stride  Gram-Schmidt workgroup stride (1: all CUs, 8: one XCD) of the
+ *              kernel-per-step form
  * 0 keeps a value.  Results are bitwise independent of all three.  A session
  * starts from the table $MLCP_HIP_TUNING (or tuning_table.txt beside the
  * library; lines "<key> <had_tile> <had_split> <gs_stride>") when it holds
